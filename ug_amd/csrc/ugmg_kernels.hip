@@ -87,29 +87,51 @@ __device__ __forceinline__ TA sell_dot(const TV *__restrict__ v, const int *__re
   return sum;
 }
 
-// b x b blocks (b = 3): out_i = sum_k sum_j A_k[i][j] x[b col_k + j] over the
-// row's entries in order, entry k's block in b*b planes of pst values;
-// chunks of 2 entries (18 values and 6 gathers in flight per lane).
+// b x b blocks: out_i = sum_k sum_j A_k[i][j] x[b col_k + j] over the row's
+// entries in order, entry k's block in b*b planes of pst values.  A row of
+// 15 to 27 blocks is a chain of rounds (columns, then values and gathers),
+// each a trip to memory, and a level has only 4 to 16 wavefronts per CU: the
+// chunk is as many entries as keep values and gathers under 96 (FP32) and
+// 144 (FP64) registers, and a chunk's columns are loaded with the chunk
+// before, so a row of 15 FP32 3x3 blocks takes two rounds.  Measured against
+// chunks of 2 (mixed solves): 65^3 elasticity 34.4 -> 23.3 ms, the locally
+// refined one 30.7 -> 23.5 ms.
 template <int B, int NT, typename TV, typename TX, typename TA>
 __device__ __forceinline__ void sell_dot_blk(const TV *__restrict__ v, size_t pst,
                                              const int *__restrict__ ci, int w,
                                              const TX *__restrict__ x, int sdo,
                                              const int *__restrict__ dtab, int rb, TA (&out)[B]) {
-  constexpr int CH = 2;
+  constexpr int CH = (sizeof(TV) == 4 ? 96 : 72) / (B * B + B) < 8 ? (sizeof(TV) == 4 ? 96 : 72) / (B * B + B) : 8;
 #pragma unroll
   for (int i = 0; i < B; ++i) out[i] = 0;
+  if (w <= 0) return;
+  const bool uni = sdo >= 0;
+  const int *__restrict__ dt = dtab + (uni ? sdo : 0);
+  int c[CH];
+  auto columns = [&](int k) {
+    if (uni) {
+#pragma unroll
+      for (int j = 0; j < CH; ++j) c[j] = rb + dt[(k + j < w) ? k + j : w - 1];
+    } else {
+#pragma unroll
+      for (int j = 0; j < CH; ++j) c[j] = ld<NT>(ci + 64 * ((k + j < w) ? k + j : w - 1));
+    }
+  };
+  columns(0);
   for (int k = 0; k < w; k += CH) {
     TV a[CH][B * B];
     TX xv[CH][B];
 #pragma unroll
     for (int j = 0; j < CH; ++j) {
       const int kk = (k + j < w) ? k + j : w - 1;
-      const int c = sdo >= 0 ? rb + dtab[sdo + kk] : ld<NT>(ci + 64 * kk);
 #pragma unroll
       for (int q = 0; q < B * B; ++q) a[j][q] = ld<NT>(v + q * pst + 64 * kk);
-#pragma unroll
-      for (int i = 0; i < B; ++i) xv[j][i] = x[(size_t)B * c + i];
     }
+#pragma unroll
+    for (int j = 0; j < CH; ++j)
+#pragma unroll
+      for (int i = 0; i < B; ++i) xv[j][i] = x[(size_t)B * c[j] + i];
+    if (k + CH < w) columns(k + CH);
 #pragma unroll
     for (int j = 0; j < CH; ++j)
       if (k + j < w) {
@@ -125,25 +147,38 @@ __device__ __forceinline__ void sell_dot_blk(const TV *__restrict__ v, size_t ps
 }
 
 // scalar weights on vectors of B components (the transfer): out_i =
-// sum_k w_k x[B col_k + i]
-template <int B, int NT, typename TV, typename TX, typename TA>
+// sum_k w_k x[B col_k + i], CH entries per round (an interpolation row has 1
+// to 4 coarse corners, a restriction row 15 to 27 fine vectors)
+template <int B, int CH, int NT, typename TV, typename TX, typename TA>
 __device__ __forceinline__ void sell_dot_diag(const TV *__restrict__ v, const int *__restrict__ ci,
                                               int w, const TX *__restrict__ x, int sdo,
                                               const int *__restrict__ dtab, int rb, TA (&out)[B]) {
-  constexpr int CH = 4;
 #pragma unroll
   for (int i = 0; i < B; ++i) out[i] = 0;
+  if (w <= 0) return;
+  const bool uni = sdo >= 0;
+  const int *__restrict__ dt = dtab + (uni ? sdo : 0);
+  int c[CH];
+  auto columns = [&](int k) {
+    if (uni) {
+#pragma unroll
+      for (int j = 0; j < CH; ++j) c[j] = rb + dt[(k + j < w) ? k + j : w - 1];
+    } else {
+#pragma unroll
+      for (int j = 0; j < CH; ++j) c[j] = ld<NT>(ci + 64 * ((k + j < w) ? k + j : w - 1));
+    }
+  };
+  columns(0);
   for (int k = 0; k < w; k += CH) {
     TV a[CH];
     TX xv[CH][B];
 #pragma unroll
-    for (int j = 0; j < CH; ++j) {
-      const int kk = (k + j < w) ? k + j : w - 1;
-      const int c = sdo >= 0 ? rb + dtab[sdo + kk] : ld<NT>(ci + 64 * kk);
-      a[j] = ld<NT>(v + 64 * kk);
+    for (int j = 0; j < CH; ++j) a[j] = ld<NT>(v + 64 * ((k + j < w) ? k + j : w - 1));
 #pragma unroll
-      for (int i = 0; i < B; ++i) xv[j][i] = x[(size_t)B * c + i];
-    }
+    for (int j = 0; j < CH; ++j)
+#pragma unroll
+      for (int i = 0; i < B; ++i) xv[j][i] = x[(size_t)B * c[j] + i];
+    if (k + CH < w) columns(k + CH);
 #pragma unroll
     for (int j = 0; j < CH; ++j)
       if (k + j < w) {
@@ -932,7 +967,7 @@ __global__ __launch_bounds__(kBlock) void k_restrict_bk(DSell<T> PT, int nsl,
     if constexpr (MAT)
       sell_dot_blk<B, NT, T, T, T>(MV(PT) + e0 + lane, PT.pst, PT.col + e0 + lane, w, bf, sdo, PT.dtab, rb, sum);
     else
-      sell_dot_diag<B, NT, T, T, T>(MV(PT) + e0 + lane, PT.col + e0 + lane, w, bf, sdo, PT.dtab, rb, sum);
+      sell_dot_diag<B, sizeof(T) == 4 ? 16 : 8, NT, T, T, T>(MV(PT) + e0 + lane, PT.col + e0 + lane, w, bf, sdo, PT.dtab, rb, sum);
     if (r >= 0) {
       const bool zero = cvnclass[r] >= 2;
       const uint32_t sk = cskip[r];
@@ -970,7 +1005,7 @@ __global__ __launch_bounds__(kBlock) void k_interp_bk(DSell<T> P, int nsl,
   if constexpr (MAT)
     sell_dot_blk<B, NT, T, T, T>(MV(P) + e0 + lane, P.pst, P.col + e0 + lane, w, cc, sdo, P.dtab, rb, sum);
   else
-    sell_dot_diag<B, NT, T, T, T>(MV(P) + e0 + lane, P.col + e0 + lane, w, cc, sdo, P.dtab, rb, sum);
+    sell_dot_diag<B, 4, NT, T, T, T>(MV(P) + e0 + lane, P.col + e0 + lane, w, cc, sdo, P.dtab, rb, sum);
   if (r < 0) return;
   const uint32_t sk = fskip[r];
 #pragma unroll
