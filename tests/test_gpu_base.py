@@ -1,7 +1,7 @@
 """Device-side EXPreProcess (np/procs/iter.cc:8685-8970): the band LU without
 pivoting (EXDecomposeMatrixDOUBLE, gm/evm.cc:1400-1418) and the explicit
 inverse from EXApplyLUDOUBLE (gm/evm.cc:1493-1510) run on the GPU during
-ugmg_preprocess (for base levels above about 2e9 multiply-adds of
+ugmg_preprocess (for base levels above about 5e7 multiply-adds of
 factorisation; UGMG_BASE_HOST=0 forces it for the small levels here).  The
 inverse is read back column by column through the
 base solve (ls over ex, one step, damp 1, on unit vectors: the GEMV returns
@@ -72,6 +72,38 @@ def test_device_base_inverse_is_bitwise_the_host_one(which):
     # and it is the inverse
     A = lv.dense()
     assert np.max(np.abs(got @ A - np.eye(n))) < 1e-10
+
+
+@pytest.mark.parametrize("n,bw", [(1, 0), (40, 1), (97, 16), (64, 31), (65, 32), (100, 33), (353, 48), (450, 420),
+                                  (700, 640), (1000, 960), (1100, 1000)])
+@pytest.mark.parametrize("ex_float", [0, 1])
+def test_device_base_band_widths(n, bw, ex_float):
+    """Every path of the factorisation and of the substitutions (panels from a
+    half bandwidth of 32 to 992, the LDS window with 32, 20 and 16 columns, the
+    general kernels outside) at the edges of its panels and chunks."""
+    rng = np.random.default_rng(n)
+    offs = sorted({o for d in {1, bw // 2, bw} for o in (-d, d) if d})
+    cols = [[v] + [v + o for o in offs if 0 <= v + o < n] for v in range(n)]
+    rp = np.concatenate([[0], np.cumsum([len(c) for c in cols])]).astype(np.int32)
+    vals = rng.uniform(-1.0, 1.0, rp[-1])
+    vals[rp[:-1]] += 8.0
+    lv = problems.Level(n=n, b=1, row_ptr=rp, col_idx=np.concatenate(cols).astype(np.int32), vals=vals,
+                        skip=np.zeros(n, np.uint32), vclass=np.full(n, 3, np.uint8), vnclass=np.zeros(n, np.uint8))
+    P = problems.Problem(dim=1, levels=[lv])
+    dev, host = (_context(P, 0, h, reorder=0, ex_float=ex_float) for h in (False, True))
+    c, b = (torch.zeros(n, dtype=torch.float64, device="cuda") for _ in range(2))
+    for u in sorted({0, n // 3, n - 17, n - 1} & set(range(n))):
+        got = []
+        for ctx in (dev, host):
+            b.zero_()
+            b[u] = 1.0
+            torch.cuda.synchronize()
+            ctx.base_solve(c, b)
+            ctx.sync()
+            got.append(c.cpu().numpy())
+        assert np.array_equal(*got)
+    dev.close()
+    host.close()
 
 
 @pytest.mark.parametrize("host_factor", [False, True])

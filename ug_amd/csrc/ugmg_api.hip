@@ -1163,8 +1163,10 @@ int launch_bcgs_iteration(ugmg_ctx *ctx, int level, bool use_iter, int restart, 
 // Host half of LmgcPreProcess (CPU only, no HIP call; safe on a worker
 // thread while the context is not otherwise used).
 // multiply-adds of the base factorisation (about n bw (bw + n)) above which
-// it runs on the device: about a second of host time
-constexpr double kBaseDeviceWork = 2.0e9;
+// it runs on the device.  Whole preprocess, host / device, the base level in
+// front: 17^2 (3e6) 1.5 / 2.0 ms, 7^3 (36e6) 4.3 / 4.4, 33^2 (84e6) 6.7 / 5.5,
+// 9^3 (187e6) 12.3 / 5.6, 11^3 59 / 13
+constexpr double kBaseDeviceWork = 5.0e7;
 
 // FULLREFINELEVEL of the levels set up to `level` (SetSurfaceClasses,
 // gm/algebra.cc:2885-2916): the lowest level holding a FINE_GRID_DOF vector
@@ -1393,6 +1395,10 @@ int factor_base_device(ugmg_ctx *ctx, HostBase &B) {
   const size_t ldx = ((size_t)n + 63) / 64 * 64;
   double *band = nullptr, *X = nullptr;
   int *pos = nullptr, *flag = nullptr;
+  // pos, lfirst and ulast behind one another
+  std::vector<int> idx(B.pos);
+  idx.insert(idx.end(), B.lfirst.begin(), B.lfirst.end());
+  idx.insert(idx.end(), B.ulast.begin(), B.ulast.end());
   auto release = [&] {
     hipFree(band);
     hipFree(X);
@@ -1401,7 +1407,7 @@ int factor_base_device(ugmg_ctx *ctx, HostBase &B) {
   };
   hipError_t e = hipMalloc((void **)&band, B.band.size() * sizeof(double));
   if (e == hipSuccess) e = hipMalloc((void **)&X, (size_t)n * ldx * sizeof(double));
-  if (e == hipSuccess) e = hipMalloc((void **)&pos, (size_t)n * sizeof(int));
+  if (e == hipSuccess) e = hipMalloc((void **)&pos, idx.size() * sizeof(int));
   if (e == hipSuccess) e = hipMalloc((void **)&flag, sizeof(int));
   if (e != hipSuccess) {
     release();
@@ -1410,10 +1416,10 @@ int factor_base_device(ugmg_ctx *ctx, HostBase &B) {
   const int zero = 0;
   e = hipMemcpyAsync(band, B.band.data(), B.band.size() * sizeof(double), hipMemcpyHostToDevice, ctx->stream);
   if (e == hipSuccess)
-    e = hipMemcpyAsync(pos, B.pos.data(), (size_t)n * sizeof(int), hipMemcpyHostToDevice, ctx->stream);
+    e = hipMemcpyAsync(pos, idx.data(), idx.size() * sizeof(int), hipMemcpyHostToDevice, ctx->stream);
   if (e == hipSuccess) e = hipMemcpyAsync(flag, &zero, sizeof(int), hipMemcpyHostToDevice, ctx->stream);
   if (e == hipSuccess) {
-    launch_base_factor(ctx->stream, band, n, B.bw, pos, X, ctx->base_inv, flag, B.fmode);
+    launch_base_factor(ctx->stream, band, B, pos, pos + n, pos + n + B.lfirst.size(), X, ctx->base_inv, flag);
     e = hipGetLastError();
   }
   int failed = 0;

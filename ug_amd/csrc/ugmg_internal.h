@@ -89,6 +89,10 @@ struct HostBase {
   bool failed = false;
   std::vector<int> order;      // BFS list order
   std::vector<int> pos;        // scalar unknown (list order) -> band position
+  // the envelope, in which elimination without pivoting fills: the first
+  // column of rows 16 q .. 16 q + 15, the last column of row i and the last
+  // row of column i of the factors
+  std::vector<int> lfirst, ulast, llast;
   std::vector<double> band;    // EX_MAT band, n (2 bw + 1) + 1 (before factoring)
   bool fmode = false;          // ex $f: FLOAT entries, LU in FLOAT arithmetic
   std::vector<double> inv;     // n x n row-major, list order (vector-major);

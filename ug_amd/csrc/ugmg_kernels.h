@@ -7,7 +7,7 @@
 #include <string>
 #include <vector>
 
-#include "ugmg_common.h"
+#include "ugmg_internal.h"
 
 namespace ugmg {
 
@@ -204,13 +204,13 @@ int assemble_device(hipStream_t st, const AsmInput &in, double *rhs, std::vector
                     AsmKeep *keep = nullptr);
 
 // Band LU (no pivoting) of the base level and its explicit inverse, on the
-// device: band (n rows, bandwidth bw, UG's EX_MAT layout) is factored in
-// place, X (n rounded up to 64, times n doubles) receives the inverse in
-// band positions as panels of 64 columns, inv (n x n) the inverse in list
+// device: band (B's; UG's EX_MAT layout) is factored in place, lfirst and
+// ulast are B's on the device, X (n rounded up to 64, times n doubles)
+// receives the inverse in band positions as panels of 64 columns, inv (n x n) the inverse in list
 // order: inv[r][u] = entry (pos[r], pos[u]).  *failed (0 on entry) is set
 // on a zero pivot.
-void launch_base_factor(hipStream_t st, double *band, int n, int bw, const int *pos, double *X,
-                        double *inv, int *failed, bool fmode = false);
+void launch_base_factor(hipStream_t st, double *band, const HostBase &B, const int *pos, const int *lfirst,
+                        const int *ulast, double *X, double *inv, int *failed);
 // inv: the rows of the dense inverse that are not unit rows (rowmap[r]: the
 // row's index there, -1 for a unit row), columns in the order cp, in FP64
 // (TI = double) or the FP32 copy for the FP32 cycle (TI = float); the

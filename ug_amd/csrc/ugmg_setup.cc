@@ -510,6 +510,33 @@ void build_base_band(const HostLevel &L, int reorder, HostBase &out, bool fmode)
   out.bw = bw;
   out.pos.resize(n);
   for (int u = 0; u < n; ++u) out.pos[u] = index[u / B] + u % B;
+  // envelope: row i of the factors starts at the row's first column and
+  // column k at the column's first row; so row i of U ends at the last
+  // column that starts at or above i, column i of L at the last row likewise
+  std::vector<int> rfirst(n), cfirst(n);
+  for (int i = 0; i < n; ++i) rfirst[i] = cfirst[i] = i;
+  for (int v = 0; v < nvec; ++v)
+    for (int m = L.rp[v]; m < L.rp[v + 1]; ++m)
+      for (int i = 0; i < B; ++i) {
+        const int w = index[L.ci[m]];
+        rfirst[index[v] + i] = std::min(rfirst[index[v] + i], w);
+        cfirst[w + i] = std::min(cfirst[w + i], index[v]);
+      }
+  out.lfirst.assign((n + 15) / 16, n);
+  out.ulast.resize(n);
+  out.llast.resize(n);
+  for (int i = 0; i < n; ++i) {
+    out.ulast[i] = out.llast[i] = i;
+    out.lfirst[i / 16] = std::min(out.lfirst[i / 16], rfirst[i]);
+  }
+  for (int i = 0; i < n; ++i) {
+    out.ulast[cfirst[i]] = std::max(out.ulast[cfirst[i]], i);
+    out.llast[rfirst[i]] = std::max(out.llast[rfirst[i]], i);
+  }
+  for (int i = 1; i < n; ++i) {
+    out.ulast[i] = std::max(out.ulast[i], out.ulast[i - 1]);
+    out.llast[i] = std::max(out.llast[i], out.llast[i - 1]);
+  }
   out.band.assign((size_t)n * (2 * (size_t)bw + 1) + 1, 0.0);
   std::vector<double> &band = out.band;
   for (int v = 0; v < nvec; ++v)
