@@ -1,0 +1,71 @@
+"""Coarse levels in one workgroup per column (k_coarse_down, k_coarse_up)
+against a launch per operation (UGMG_FUSE_ROWS=0): the same bits, for both
+smoothers and precisions, several columns, step counts, c += (the second
+cycle of a mixed step), levels at and past the limit and local levels whose
+coarse vectors keep their value in the restriction."""
+import numpy as np
+import pytest
+
+from ug_amd import problems, ugmg
+
+pytestmark = pytest.mark.gpu
+
+torch = pytest.importorskip("torch")
+
+
+def _cycle(P, monkeypatch, rows, cols=1, cycles=1, **kw):
+    if rows is None:
+        monkeypatch.delenv("UGMG_FUSE_ROWS", raising=False)
+    else:
+        monkeypatch.setenv("UGMG_FUSE_ROWS", str(rows))
+    lv = P.levels[-1]
+    ctx = ugmg.Context(0)
+    ctx.set_hierarchy(P)
+    prm = dict(nu1=2, nu2=2, gamma=1, baselevel=1, smoother=ugmg.SMOOTH_GS, damp=1.0, base_abslimit=1e-300,
+               base_maxiter=1)
+    prm.update(kw)
+    ctx.set_params(**prm)
+    if cols > 1:
+        ctx.set_batch(cols)
+    ctx.preprocess()
+    b = torch.from_numpy(np.random.default_rng(3).uniform(-1.0, 1.0, (cols, lv.n))).cuda()
+    b[:, torch.from_numpy(lv.skip & 1 == 1).cuda()] = 0.0
+    c = torch.zeros_like(b)
+    torch.cuda.synchronize()
+    for _ in range(cycles):
+        if cols > 1:
+            ctx.iter_batch(P.top, c, b)
+        else:
+            ctx.iter(P.top, c[0], b[0])
+    ctx.sync()
+    ctx.close()
+    return c.cpu().numpy(), b.cpu().numpy()
+
+
+CASES = [
+    ("2d", lambda: problems.q1(2, 3, 5, problems.KAPPA_JUMP, seed=1), dict(smoother=ugmg.SMOOTH_JAC, damp=0.8, nu1=1, nu2=3)),
+    ("2d", lambda: problems.q1(2, 2, 5, problems.KAPPA_ONE, seed=2), dict(baselevel=0, damp=0.9, precision=ugmg.MIXED)),
+    ("3d", lambda: problems.q1(3, 1, 5, problems.KAPPA_JUMP, seed=3), dict(nu1=0, nu2=2)),
+    ("3d", lambda: problems.q1(3, 3, 3, problems.KAPPA_JUMP, seed=4), dict(baselevel=2, nu1=3, nu2=1, precision=ugmg.MIXED,
+                                                                          inner_cycles=2)),
+    ("3d cols", lambda: problems.q1(3, 1, 4, problems.KAPPA_JUMP, seed=5), dict(cols=3)),
+    ("3d jac", lambda: problems.q1(3, 1, 4, problems.KAPPA_JUMP, seed=6), dict(smoother=ugmg.SMOOTH_JAC, damp=0.8, cols=2,
+                                                                              nu2=0)),
+    ("3d below", lambda: problems.q1(3, 1, 5, problems.KAPPA_JUMP, seed=8), dict(precision=ugmg.MIXED, inner_cycles=2,
+                                                                                cycles=3)),
+    ("p1", lambda: problems.p1_cd(5, 1e-3, float("nan"), seed=7), dict(cycles=2)),
+    ("local", lambda: problems.p1_local(3, 3), dict(cycles=2)),
+    ("local jac", lambda: problems.p1_local(4, 2), dict(smoother=ugmg.SMOOTH_JAC, damp=0.8, cycles=2)),
+]
+
+
+@pytest.mark.parametrize("k", range(len(CASES)))
+def test_coarse_levels_are_bitwise_the_separate_launches(k, monkeypatch):
+    tag, make, kw = CASES[k]
+    P = make()
+    print(f"coarse {k} {tag} {[lv.n for lv in P.levels]}", flush=True)
+    want = _cycle(P, monkeypatch, 0, **kw)
+    assert np.all(np.isfinite(want[0])) and np.any(want[0])
+    for rows in (None, P.levels[-2].n, P.levels[-2].n - 1):
+        got = _cycle(P, monkeypatch, rows, **kw)
+        assert np.array_equal(got[0], want[0]) and np.array_equal(got[1], want[1]), rows

@@ -264,8 +264,9 @@ struct ugmg_ctx {
   double *surf_sq = nullptr;
   double *surf_sq_host = nullptr;
   int surf_sq_host_cap = 0;
-  // levels bl..fuse_top run inside one fused coarse-cycle kernel
-  int fuse_top = -1;
+  // levels bl + 1..fuse_top of an FP64 [0] and FP32 [1] cycle run in one
+  // workgroup per column (k_coarse_down, k_coarse_up)
+  int fuse_top[2] = {-1, -1};
   CLevel<double> *clev64 = nullptr;
   CLevel<float> *clev32 = nullptr;
   // base solver: partial sums of the base defect norm, first norm
@@ -442,7 +443,7 @@ void free_device(ugmg_ctx *ctx) {
   ctx->base_cpos = nullptr;
   ctx->clev64 = nullptr;
   ctx->clev32 = nullptr;
-  ctx->fuse_top = -1;
+  ctx->fuse_top[0] = ctx->fuse_top[1] = -1;
   ctx->base_part = nullptr;
   ctx->base_first = nullptr;
   ctx->part = nullptr;
@@ -631,36 +632,34 @@ void post_smooth_folded(ugmg_ctx *ctx, int l, const T *t, T *b, T *c, int nsteps
   smooth<T>(ctx, l, u, b, c, 1, nsteps, 1, true);
 }
 
-BaseArgs base_args(ugmg_ctx *ctx) {
-  BaseArgs ba;
-  ba.n = ctx->dev[ctx->bl].n;
-  ba.maxiter = ctx->p.base_maxiter;
-  ba.failed = ctx->base.failed ? 1 : 0;
-  ba.damp = ctx->p.base_damp[0];
-  ba.abslimit = ctx->p.base_abslimit[0];
-  ba.red = ctx->p.base_red[0];
-  ba.inv = ctx->base_inv;
-  return ba;
+// does a cycle run level l in k_coarse_down and k_coarse_up?
+template <typename T>
+bool in_coarse(const ugmg_ctx *ctx, int l) {
+  return l > ctx->bl && l <= ctx->fuse_top[std::is_same_v<T, double> ? 0 : 1] && ctx->p.gamma == 1;
 }
 
-// Lmgc on levels top..bl in one workgroup (levels at most a few thousand
-// vectors, where a separate launch per operation would be latency bound)
+// levels top..bl + 1 of a cycle before (up = false) or after the base solve
 template <typename T>
-void coarse_cycle(ugmg_ctx *ctx, int top, T *c, T *b, int cmode) {
+void coarse_levels(ugmg_ctx *ctx, int top, T *c, T *b, int cmode, bool up) {
   CoarseArgs<T> a;
   if constexpr (std::is_same_v<T, double>) a.lv = ctx->clev64;
   else a.lv = ctx->clev32;
+  const ugmg_params &p = ctx->p;
   a.bl = ctx->bl;
   a.top = top;
-  const ugmg_params &p = ctx->p;
-  a.cp = CycleParams{p.nu1, p.nu2, p.gamma, p.smoother, p.damp[0], p.lmgc_damp[0]};
-  a.base = base_args(ctx);
-  a.baseA = ctx->dev[ctx->bl].A.d64();
-  a.base_vclass = ctx->dev[ctx->bl].vclass;
+  a.smoother = sm_kind(ctx, up) == UGMG_SMOOTH_GS ? 1 : 0;
+  a.nu = up ? p.nu2 : p.nu1;
+  a.damp = (T)sm_damp(ctx, up)[0];
+  a.lmgc_damp = (T)p.lmgc_damp[0];
   a.c_top = c;
   a.b_top = b;
-  a.cmode_top = cmode;
-  launch_coarse_cycle<T>(ctx->stream, a, ctx->dev[ctx->bl].n);
+  a.cmode = cmode;
+  a.nmax = a.ncmax = 0;
+  for (int l = ctx->bl; l <= top; ++l) {
+    if (l > ctx->bl) a.nmax = std::max(a.nmax, ctx->dev[l].n);
+    if (l < top) a.ncmax = std::max(a.ncmax, ctx->dev[l].n);
+  }
+  launch_coarse<T>(ctx->stream, a, up, ctx->nb);
 }
 
 // ls over ex on the base level: `maxiter` GEMVs with the dense inverse.  The
@@ -732,25 +731,34 @@ template <typename T>
 void lmgc(ugmg_ctx *ctx, int l, T *c, T *b, int cmode, bool c0_done = false) {
   const ugmg_params &p = ctx->p;
   hipStream_t st = ctx->stream;
-  if (l <= ctx->fuse_top && ctx->nb == 1) {
-    coarse_cycle<T>(ctx, l, c, b, cmode);
-    return;
-  }
   if (l <= ctx->bl) {
     base_solve<T>(ctx, c, b, cmode, false, true);
     return;
   }
+  const bool coarse = in_coarse<T>(ctx, l);
+  const int nb = ctx->nb;
+  T *ctop = c, *btop = b;
+  const int top = l;
+  if (coarse) {
+    coarse_levels<T>(ctx, l, c, b, cmode, false);
+    if (l > ctx->bl + 1) {
+      l = ctx->bl + 1;
+      c = ctx->dev[l].cv<T>();
+      b = ctx->dev[l].bv<T>();
+    }
+  }
   DevLevel &d = ctx->dev[l];
   DevLevel &dc = ctx->dev[l - 1];
   T *t = d.tv<T>();
-  const int nb = ctx->nb;
-  smooth<T>(ctx, l, t, b, c, cmode, p.nu1, c0_done ? 1 : 0);
-  if (p.nu1 == 0 && cmode == 0) launch_fill<T>(st, d.n, c, (T)0, batch(ctx, l));
+  if (!coarse) {
+    smooth<T>(ctx, l, t, b, c, cmode, p.nu1, c0_done ? 1 : 0);
+    if (p.nu1 == 0 && cmode == 0) launch_fill<T>(st, d.n, c, (T)0, batch(ctx, l));
+  }
   // RestrictDefect(level, b, b, Factor_One); on a coarse level that runs
-  // lmgc below (not the base solve or the fused coarse cycle) also its
-  // first pre-smoothing sweep's colour 0
-  const bool to_base = l - 1 == ctx->bl && (ctx->fuse_top < ctx->bl || nb > 1);
-  const bool pre0 = l - 1 > ctx->bl && l - 1 > ctx->fuse_top && p.gamma >= 1 &&
+  // lmgc below (not the base solve or k_coarse_down) also its first
+  // pre-smoothing sweep's colour 0
+  const bool to_base = l - 1 == ctx->bl;
+  const bool pre0 = l - 1 > ctx->bl && !in_coarse<T>(ctx, l - 1) && p.gamma >= 1 &&
                     fold_colour0(ctx, l - 1, p.nu1);
   // onto the base level (scalar) also b in the inverse's column order, into
   // the base level's spare vector u, for the first base iteration.  With
@@ -775,6 +783,10 @@ void lmgc(ugmg_ctx *ctx, int l, T *c, T *b, int cmode, bool c0_done = false) {
     } else {
       lmgc<T>(ctx, l - 1, dc.cv<T>(), dc.bv<T>(), g == 0 ? 0 : 1, g == 0 && pre0);
     }
+  }
+  if (coarse) {
+    coarse_levels<T>(ctx, top, ctop, btop, 1, true);
+    return;
   }
   // InterpolateCorrection(level, t, c, damp); dadd(c, t); dmatmul_minus(b, A, t)
   if (per_comp(ctx, p.lmgc_damp)) {   // damp per component: dscalx after the sum
@@ -1003,17 +1015,16 @@ double base_bytes(const ugmg_ctx *ctx, int sv, bool restricted, bool need_b) {
   return by;
 }
 
-// one lmgc cycle as lmgc() issues it (the fused coarse-cycle kernel, an
-// opt-in for tiny hierarchies, is not modelled and counts 0)
+// one lmgc cycle as lmgc() issues it; levels in k_coarse_down and
+// k_coarse_up count as the separate launches would
 double lmgc_bytes(const ugmg_ctx *ctx, int l, int sv, int cmode, bool c0_done) {
   const ugmg_params &p = ctx->p;
-  if (l <= ctx->fuse_top) return 0.0;
   if (l <= ctx->bl) return base_bytes(ctx, sv, false, true) + vbytes(ctx->dev[l], sv) + ctx->dev[l].n;
   const DevLevel &d = ctx->dev[l], &dc = ctx->dev[l - 1];
   double by = smooth_bytes(ctx, l, sv, cmode, p.nu1, c0_done ? 1 : 0);
   if (p.nu1 == 0 && cmode == 0) by += vbytes(d, sv);
-  const bool to_base = l - 1 == ctx->bl && ctx->fuse_top < ctx->bl;
-  const bool pre0 = l - 1 > ctx->bl && l - 1 > ctx->fuse_top && p.gamma >= 1 && fold_colour0(ctx, l - 1, p.nu1);
+  const bool to_base = l - 1 == ctx->bl;
+  const bool pre0 = l - 1 > ctx->bl && p.gamma >= 1 && fold_colour0(ctx, l - 1, p.nu1);
   by += op_bytes(ctx, l, Op::Restrict, sv);
   if (pre0) by += dc.n + (double)dc.color_rows[0] * 2.0 * sv;
   if (to_base && ctx->nb == 1 && ctx->base_cpos && !ctx->base.failed && !dc.vt &&
@@ -1168,6 +1179,9 @@ int launch_bcgs_iteration(ugmg_ctx *ctx, int level, bool use_iter, int restart, 
 // 9^3 (187e6) 12.3 / 5.6, 11^3 59 / 13
 constexpr double kBaseDeviceWork = 5.0e7;
 
+// the largest level that k_coarse_down and k_coarse_up take
+constexpr int kCoarseRows = 12288;
+
 // FULLREFINELEVEL of the levels set up to `level` (SetSurfaceClasses,
 // gm/algebra.cc:2885-2916): the lowest level holding a FINE_GRID_DOF vector
 // (VCLASS >= 2, VNCLASS <= 1); `level` when there is none
@@ -1303,7 +1317,7 @@ int prep_host(ugmg_ctx *ctx, int level, PrepState &ps) {
   const char *env_split = std::getenv("UGMG_GS_SPLIT");
   ctx->gs_split = !(env_split && std::atoi(env_split) == 0);
   const char *env_fuse = std::getenv("UGMG_FUSE_ROWS");
-  ps.fuse_rows = env_fuse ? std::atoi(env_fuse) : 0;
+  ps.fuse_rows = env_fuse ? std::atoi(env_fuse) : kCoarseRows;
   ps.level = level;
   ps.bl = bl;
   // UGMG_GS_WINDOW: window of the GS device order (unset: chosen per level;
@@ -1722,27 +1736,33 @@ int prep_device(ugmg_ctx *ctx, PrepState &ps) {
         HIPCHK(hipStreamSynchronize(ctx->stream));
       }
     }
-    // fused coarse levels (opt-in): the base level and every level above it
-    // up to fuse_rows vectors (and at most kMaxColors colours)
-    ctx->fuse_top = -1;
     if (ctx->grouped) {
       size_t mx = 1;
       for (int l = bl; l <= level; ++l) mx = std::max(mx, ctx->host[l].a.size());
       if ((rc = dalloc(ctx, &ctx->stage, mx))) return rc;
     }
-    if (ps.fuse_rows > 0 && ctx->dev[bl].n <= 2048 && ctx->b == 1 && !ctx->grouped && ps.ntypes == 1 &&
-        !split_smoothers(ctx->p) && ctx->p.base_iter == UGMG_BASE_EX) {
-      ctx->fuse_top = bl;
+    // coarse levels in one workgroup per column: those above the base level
+    // up to the first that does not fit its LDS (at most fuse_rows vectors)
+    for (int f32 = 0; f32 < 2; ++f32) {
+      int &ft = ctx->fuse_top[f32];
+      ft = bl;
+      if (ctx->b != 1 || ps.ntypes != 1) continue;
+      size_t nmax = 0, ncmax = 0;
       for (int l = bl + 1; l <= level; ++l) {
-        if (ctx->dev[l].n > ps.fuse_rows || ctx->dev[l].ncolors > kMaxColors) break;
-        ctx->fuse_top = l;
+        nmax = std::max(nmax, (size_t)ctx->dev[l].n);
+        ncmax = std::max(ncmax, (size_t)ctx->dev[l - 1].n);
+        if (ctx->dev[l].n > ps.fuse_rows || ctx->dev[l].ncolors > kMaxColors ||
+            (3 * nmax + ncmax) * (f32 ? sizeof(float) : sizeof(double)) > kCoarseLds)
+          break;
+        ft = l;
       }
     }
     ctx->base_b_dead = true;
     for (uint8_t v : ctx->host[bl].vnc) ctx->base_b_dead &= v >= 2;
-    std::vector<CLevel<double>> c64(std::max(ctx->fuse_top + 1, 1));
-    std::vector<CLevel<float>> c32(std::max(ctx->fuse_top + 1, 1));
-    for (int l = bl; l <= ctx->fuse_top; ++l) {
+    const int ft = std::max(ctx->fuse_top[0], ctx->fuse_top[1]);
+    std::vector<CLevel<double>> c64(ft + 1);
+    std::vector<CLevel<float>> c32(ft + 1);
+    for (int l = bl; l <= ft; ++l) {
       const DevLevel &D = ctx->dev[l];
       auto fill = [&](auto &C, auto tag) {
         using T = decltype(tag);
@@ -1760,9 +1780,11 @@ int prep_device(ugmg_ctx *ctx, PrepState &ps) {
         C.vclass = D.vclass;
         C.vnclass = D.vnclass;
         C.skip = D.skip;
+        C.iskip = D.iskip;
         C.c = D.cv<T>();
         C.b = D.bv<T>();
-        C.t = D.tv<T>();
+        C.vs = D.vs;
+        C.dms = D.dms;
       };
       fill(c64[l], double());
       fill(c32[l], float());

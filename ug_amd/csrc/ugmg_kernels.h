@@ -43,18 +43,7 @@ struct DSell {
   int bb = 1;
 };
 
-// base-level solver settings: ls($m,$red,$abslimit) over ex($damp)
-struct BaseArgs {
-  int n;
-  int maxiter;
-  int failed;
-  double damp;
-  double abslimit;
-  double red;
-  const double *inv;   // n x n, row-major
-};
-
-// one level as seen by the fused coarse-cycle kernel
+// a level as k_coarse_down and k_coarse_up see it
 template <typename T>
 struct CLevel {
   int n;
@@ -63,26 +52,24 @@ struct CLevel {
   DSell<T> A, L, U, P, PT;   // P: interpolation from l-1, PT: restriction to l-1
   const T *diag;
   const uint8_t *vclass, *vnclass;
-  const uint32_t *skip;
-  T *c, *b, *t;
+  const uint32_t *skip, *iskip;
+  T *c, *b;
+  size_t vs, dms;            // column strides of the vectors and of the diagonal
 };
 
-struct CycleParams {
-  int nu1, nu2, gamma, smoother;
-  double damp, lmgc_damp;
-};
-
+// levels top .. bl + 1 of a cycle on one side of the base solve
 template <typename T>
 struct CoarseArgs {
   const CLevel<T> *lv;   // device array indexed by level
   int bl, top;
-  CycleParams cp;
-  BaseArgs base;
-  DSell<double> baseA;   // FP64 copy of the base-level matrix
-  const uint8_t *base_vclass;
+  int smoother, nu;      // 0 Jacobi, 1 multicolour GS; steps per level
+  T damp, lmgc_damp;
   T *c_top, *b_top;
-  int cmode_top;         // 0: c := correction, 1: c += correction
+  int cmode;             // down: 0: c_top := correction, 1: c_top += correction
+  int nmax, ncmax;       // vectors of the largest level, and of the largest below one
 };
+// LDS of a workgroup: three vectors of a level and one of the level below
+constexpr size_t kCoarseLds = 160 * 1024;
 
 // Batched launches: every vector argument holds `nrhs` columns, column j at
 // offset j * vs (vs = the level's column stride, >= n); the column index of a
@@ -276,7 +263,7 @@ template <typename TD, typename TS>
 void launch_scatter(hipStream_t st, int n, const int *perm, const TS *s, TD *d, int nrhs,
                     size_t vss, size_t vsd, int b);
 template <typename T>
-void launch_coarse_cycle(hipStream_t st, const CoarseArgs<T> &args, int base_n);
+void launch_coarse(hipStream_t st, const CoarseArgs<T> &args, bool up, int nrhs);
 // coarse values ca (pattern crp/cci, bb values per entry) = P^T A P; pt*:
 // every fine vector that interpolates from coarse row I, in list order
 // *bad = min(*bad, first vector of class >= 3 whose diagonal block

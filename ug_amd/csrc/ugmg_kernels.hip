@@ -46,13 +46,13 @@ __device__ __forceinline__ T ld(const T *p) {
 // Uniform slice (sdo >= 0): col_k = rb + dtab[sdo + k] (wave-uniform offsets
 // in scalar registers), so the x gathers issue together with the value loads;
 // explicit slice: col_k = ci[64 k].  TA is the accumulation type.
-template <int CH, int NT, typename TV, typename TX, typename TA>
+template <int CH, int NT, typename TV, typename TX, typename TA, typename DT>
 __device__ __forceinline__ TA sell_dot(const TV *__restrict__ v, const int *__restrict__ ci,
                                        int w, const TX *__restrict__ x, int sdo,
-                                       const int *__restrict__ dtab, int rb) {
+                                       const DT *dtab, int rb) {
   TA sum = 0;
   if (sdo >= 0) {
-    const int *__restrict__ dt = dtab + sdo;
+    const DT *dt = dtab + sdo;
     for (int k = 0; k < w; k += CH) {
       TV a[CH];
       TX xv[CH];
@@ -546,8 +546,7 @@ __global__ __launch_bounds__(BS) void k_gs_color_fused(DSell<TV> L, DSell<TV> U,
   if (r < 0) return;
   const T bn = br - damp * (br + su);
   b[o + r] = bn;
-  const T t = damp * vo;
-  c[o + r] = CMODE == 0 ? t : cr + t;
+  c[o + r] = CMODE == 0 ? damp * vo : fma(damp, vo, cr);
   v[r] = (bn - sl) / dr;
 }
 
@@ -595,8 +594,7 @@ __global__ __launch_bounds__(2 * kSlice) void k_gs_color_fused2(DSell<TV> L, DSe
   if (half == 1 || r < 0) return;
   const T bn = br - damp * (br + part);
   b[o + r] = bn;
-  const T t = damp * vo;
-  c[o + r] = CMODE == 0 ? t : cr + t;
+  c[o + r] = CMODE == 0 ? damp * vo : fma(damp, vo, cr);
   v[r] = (bn - lsum[lane]) / dr;
 }
 
@@ -625,12 +623,9 @@ __global__ __launch_bounds__(kBlock) void k_gs_defect(DSell<TV> U, int nsl,
   const T sum = sell_dot<MW, NT, TV, T, T>(MV(U) + e0 + lane, U.col + e0 + lane, w, v, sdo, U.dtab, rb);
   if (r < 0) return;
   b[o + r] = act ? br - damp * (br + sum) : br - damp * sum;
-  const T t = damp * vr;
-  if (c) {
-    if (CMODE == 0) c[o + r] = t;
-    else c[o + r] = cr + t;
-  }
-  if (xout) xout[o + r] = t;
+  // (the rounding of c is that of the folded sweeps)
+  if (c) c[o + r] = CMODE == 0 ? damp * vr : fma(damp, vr, cr);
+  if (xout) xout[o + r] = damp * vr;
 }
 
 // --------------------------------------------------------------- transfer
@@ -1301,173 +1296,174 @@ void launch_galerkin(hipStream_t st, int nc, int bb, const int *ptp, const int *
     k_galerkin<1><<<(nc + kBlock - 1) / kBlock, kBlock, 0, st>>>(nc, ptp, pti, ptw, frp, fci, fa, pp, pi, pw, crp, cci, ca);
 }
 
-// ==================================================== fused coarse cycle
-// One workgroup runs Lmgc on every level from `top` down to the base level:
-// each operation is a loop over rows or slabs followed by a workgroup
-// barrier, so the levels below a few thousand vectors cost one launch per
-// cycle instead of dozens of latency-bound launches.
-
-__device__ __forceinline__ double wg_sum(double s, double *red) {
-  for (int off = 32; off > 0; off >>= 1) s += __shfl_down(s, off, 64);
-  __syncthreads();
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
-  __syncthreads();
-  double t = 0.0;
-  for (int i = 0; i < kCoarseThreads / 64; ++i) t += red[i];
-  return t;
+// ======================================================== coarse levels
+// The levels above the base level that fit one CU's LDS: one workgroup per
+// column runs everything a cycle does on them before the base solve
+// (k_coarse_down: smoothing and restriction, top to bl + 1) and after it
+// (k_coarse_up: interpolation, defect, smoothing).  A launch per operation
+// costs 2.3 to 3.5 us on these levels, of which 1.6 us are the launch itself
+// and the rest the chain kernel arguments -> slice header -> entries ->
+// gather; here an operation ends in a workgroup barrier, the vectors are in
+// LDS, and headers stay in the scalar cache.  The workgroup reads the slabs
+// through one CU (about 64 bytes a cycle), which bounds the larger levels.
+// Every row is formed as in the separate kernels, in the same order: the
+// same bits.  V(1,1) Jacobi cycle on 65^2 from 117 to 57 us.
+//
+// The kernels store between their passes, so what they read through level
+// and slab pointers would be loaded per lane; it does not change while they
+// run and is read as constant memory.
+template <typename U>
+using constant = const U __attribute__((address_space(4)));
+template <typename U>
+__device__ __forceinline__ U cld(const U &p) {
+  return *(constant<U> *)(uintptr_t)&p;
 }
 
-template <typename TV, typename TX, class Epi>
-__device__ __forceinline__ void wg_sell(const DSell<TV> &S, int s0, int s1,
-                                        const TX *__restrict__ x, Epi epi) {
-  const int nslot = (s1 - s0) * kSlice;
-  for (int slot = threadIdx.x; slot < nslot; slot += kCoarseThreads) {
-    const int s = __builtin_amdgcn_readfirstlane(s0 + (slot >> 6));
-    const int lane = slot & 63;
-    const int r = S.rows[s * kSlice + lane];
-    const int e0 = S.soff[s], w = (S.soff[s + 1] - e0) >> 6;
-    const int sdo = S.sdoff[s];
-    const int rb = r >= 0 ? r : S.rows[s * kSlice];
-    const TX sum = sell_dot<8, 0, TV, TX, TX>(S.val + e0 + lane, S.col + e0 + lane, w, x, sdo, S.dtab, rb);
-    if (r >= 0) epi(r, sum);
+template <typename T, class Pre, class Epi>
+__device__ __forceinline__ void wg_slices(const DSell<T> &S, int col_, int s0, int s1, const T *x, Pre pre,
+                                          Epi epi) {
+  const int lane = threadIdx.x & 63;
+  const T *__restrict__ val = cld(S.val) + cld(S.mst) * (size_t)col_;
+  const int *__restrict__ rows = cld(S.rows), *__restrict__ col = cld(S.col);
+  constant<int> *soff = (constant<int> *)(uintptr_t)cld(S.soff), *sdoff = (constant<int> *)(uintptr_t)cld(S.sdoff),
+                *dtab = (constant<int> *)(uintptr_t)cld(S.dtab), *rows0 = (constant<int> *)(uintptr_t)rows;
+  for (int q = s0 + (int)(threadIdx.x >> 6); q < s1; q += kCoarseThreads / 64) {
+    const int s = __builtin_amdgcn_readfirstlane(q);
+    const int r = rows[s * kSlice + lane];
+    const int e0 = soff[s], w = (soff[s + 1] - e0) >> 6;
+    const int sdo = sdoff[s];
+    const int rb = r >= 0 ? r : rows0[s * kSlice];
+    const auto own = pre(rb);                 // the row's own data load alongside the entries
+    const T *v = val + e0 + lane;
+    const int *ci = col + e0 + lane;
+    T sum;
+    if (w <= 8) sum = sell_dot<8, 0, T, T, T>(v, ci, w, x, sdo, dtab, rb);
+    else if (w <= 16) sum = sell_dot<16, 0, T, T, T>(v, ci, w, x, sdo, dtab, rb);
+    else sum = sell_dot<14, 0, T, T, T>(v, ci, w, x, sdo, dtab, rb);   // 27: two rounds
+    if (r >= 0) epi(r, sum, own);
   }
-  __syncthreads();
-}
-
-// ls over ex on the base level: first = |b|; converged = first < abslimit;
-// repeat m: x = damp inv b; b -= A x; c += x; stop on abslimit or red.
-template <typename T>
-__device__ void wg_base_solve(const BaseArgs &ba, const DSell<double> &A,
-                              const uint8_t *__restrict__ vclass, T *__restrict__ b,
-                              T *__restrict__ c, int cmode, double *sh, double *red) {
-  const int n = ba.n;
-  double *bl = sh, *xl = sh + n, *cl = sh + 2 * n;
-  const int tid = threadIdx.x;
-  for (int i = tid; i < n; i += kCoarseThreads) {
-    bl[i] = (double)b[i];
-    cl[i] = cmode ? (double)c[i] : 0.0;
-  }
-  __syncthreads();
-  auto norm = [&]() {
-    double s = 0.0;
-    for (int i = tid; i < n; i += kCoarseThreads)
-      if (vclass[i] >= 2) s += bl[i] * bl[i];
-    return sqrt(wg_sum(s, red));
-  };
-  const double first = norm();
-  double target = first * ba.red;
-  if (target == 0.0) target = ba.red;
-  bool conv = fabs(first) < fabs(ba.abslimit);
-  for (int it = 0; it < ba.maxiter && !conv && !ba.failed; ++it) {
-    // x = damp * inv b: one wavefront per row, lanes across the columns
-    const int wave = tid >> 6, lane = tid & 63;
-    for (int i = wave; i < n; i += kCoarseThreads / 64) {
-      const double *row = ba.inv + (size_t)i * n;
-      double s = 0.0;
-      for (int j = lane; j < n; j += 64) s += row[j] * bl[j];
-      for (int off = 32; off > 0; off >>= 1) s += __shfl_down(s, off, 64);
-      if (lane == 0) xl[i] = s * ba.damp;
-    }
-    __syncthreads();
-    wg_sell(A, 0, A.nslices, xl, [&](int r, double s) { bl[r] -= s; });
-    for (int i = tid; i < n; i += kCoarseThreads) cl[i] += xl[i];
-    const double last = norm();
-    conv = fabs(last) < fabs(ba.abslimit) || fabs(last) < fabs(target);
-  }
-  __syncthreads();
-  for (int i = tid; i < n; i += kCoarseThreads) {
-    b[i] = (T)bl[i];
-    c[i] = (T)cl[i];
-  }
-  __syncthreads();
 }
 
 template <typename T>
-__device__ void wg_smooth(const CLevel<T> &L, const CycleParams &cp, T *__restrict__ c,
-                          T *__restrict__ b, int cmode) {
-  const T damp = (T)cp.damp;
-  T *__restrict__ t = L.t;
-  if (cp.smoother == 0) {
-    for (int i = threadIdx.x; i < L.n; i += kCoarseThreads)
-      t[i] = L.vclass[i] < 3 ? (T)0 : (b[i] / L.diag[i]) * damp;
-    __syncthreads();
-    wg_sell(L.A, 0, L.A.nslices, t, [&](int r, T s) {
-      b[r] -= s;
-      if (cmode) c[r] += t[r];
-      else c[r] = t[r];
-    });
-  } else {
-    for (int k = 0; k < L.ncolors; ++k)
-      wg_sell(L.L, L.color_slices[k], L.color_slices[k + 1], t, [&](int r, T s) {
-        t[r] = L.vclass[r] < 3 ? (T)0 : (b[r] - s) / L.diag[r];
+struct DiagClass {
+  T d;
+  bool act;
+};
+
+// nu smoothing steps on t, b, c (LDS); cmode: correction mode of the first
+template <typename T>
+__device__ __forceinline__ void wg_smooth(const CLevel<T> &L, int col_, int smoother, T damp, int nu, int cmode,
+                                          T *t, T *b, T *c) {
+  const T *__restrict__ diag = cld(L.diag) + cld(L.dms) * (size_t)col_;
+  const uint8_t *__restrict__ vclass = cld(L.vclass);
+  const int n = cld(L.n), ncolors = cld(L.ncolors);
+  auto none = [](int) { return 0; };
+  for (int i = 0; i < nu; ++i) {
+    const bool set = i == 0 && cmode == 0;
+    if (smoother == 0) {
+      for (int r = threadIdx.x; r < n; r += kCoarseThreads)
+        t[r] = vclass[r] < 3 ? (T)0 : (b[r] / diag[r]) * damp;
+      __syncthreads();
+      wg_slices(L.A, col_, 0, cld(L.A.nslices), t, none, [&](int r, T s, int) {
+        b[r] -= s;
+        c[r] = set ? t[r] : c[r] + t[r];
       });
-    wg_sell(L.U, 0, L.U.nslices, t, [&](int r, T s) {
-      const T br = b[r];
-      b[r] = L.vclass[r] >= 3 ? br - damp * (br + s) : br - damp * s;
-      const T tt = damp * t[r];
-      if (cmode) c[r] += tt;
-      else c[r] = tt;
-    });
-  }
-}
-
-template <typename T>
-__global__ __launch_bounds__(kCoarseThreads) void k_coarse_cycle(CoarseArgs<T> a) {
-  extern __shared__ double sh[];
-  __shared__ double red[kCoarseThreads / 64];
-  const CycleParams cp = a.cp;
-  int phase[kMaxLevels], gcount[kMaxLevels], cm[kMaxLevels];
-  int l = a.top;
-  phase[l] = 0;
-  cm[l] = a.cmode_top;
-  while (l <= a.top) {
-    const CLevel<T> &L = a.lv[l];
-    T *c = l == a.top ? a.c_top : L.c;
-    T *b = l == a.top ? a.b_top : L.b;
-    if (l <= a.bl) {
-      wg_base_solve<T>(a.base, a.baseA, a.base_vclass, b, c, cm[l], sh, red);
-      ++l;
+      __syncthreads();
       continue;
     }
-    const CLevel<T> &C = a.lv[l - 1];
-    if (phase[l] == 0) {
-      for (int i = 0; i < cp.nu1; ++i) wg_smooth<T>(L, cp, c, b, i == 0 ? cm[l] : 1);
-      if (cp.nu1 == 0 && cm[l] == 0) {
-        for (int i = threadIdx.x; i < L.n; i += kCoarseThreads) c[i] = (T)0;
-        __syncthreads();
-      }
-      wg_sell(L.PT, 0, L.PT.nslices, b, [&](int I, T s) {
-        const T base = C.vnclass[I] >= 2 ? (T)0 : C.b[I];
-        C.b[I] = (C.skip[I] & 1u) ? base : base + s;
-      });
-      gcount[l] = 0;
-      phase[l] = 1;
-      if (cp.gamma > 0) {
-        --l;
-        phase[l] = 0;
-        cm[l] = 0;
-        continue;
-      }
-      for (int i = threadIdx.x; i < C.n; i += kCoarseThreads) C.c[i] = (T)0;
+    for (int k = 0; k < ncolors; ++k) {
+      wg_slices(L.L, col_, cld(L.color_slices[k]), cld(L.color_slices[k + 1]), t,
+                [&](int r) { return DiagClass<T>{diag[r], vclass[r] >= 3}; },
+                [&](int r, T s, const DiagClass<T> &o) { t[r] = o.act ? (b[r] - s) / o.d : (T)0; });
       __syncthreads();
-    } else {
-      if (++gcount[l] < cp.gamma) {
-        --l;
-        phase[l] = 0;
-        cm[l] = 1;
-        continue;
-      }
     }
-    const T ld = (T)cp.lmgc_damp;
-    wg_sell(L.P, 0, L.P.nslices, C.c, [&](int v, T s) {
-      const T tv = (L.skip[v] & 1u) ? (T)0 : ld * s;
-      L.t[v] = tv;
-      c[v] += tv;
-    });
-    wg_sell(L.A, 0, L.A.nslices, L.t, [&](int r, T s) { b[r] -= s; });
-    for (int i = 0; i < cp.nu2; ++i) wg_smooth<T>(L, cp, c, b, 1);
-    if (l == a.top) break;
-    ++l;
+    wg_slices(L.U, col_, 0, cld(L.U.nslices), t, [&](int r) { return vclass[r] >= 3; },
+              [&](int r, T s, bool act) {
+                const T br = b[r];
+                b[r] = act ? br - damp * (br + s) : br - damp * s;
+                c[r] = set ? damp * t[r] : fma(damp, t[r], c[r]);
+              });
+    __syncthreads();
+  }
+}
+
+template <typename T>
+__device__ __forceinline__ void wg_copy(int n, T *dst, const T *src) {
+  for (int i = threadIdx.x; i < n; i += kCoarseThreads) dst[i] = src[i];
+}
+
+template <typename T>
+__global__ __launch_bounds__(kCoarseThreads) void k_coarse_down(CoarseArgs<T> a) {
+  extern __shared__ double sh[];
+  T *t = (T *)sh, *b = t + a.nmax, *c = b + a.nmax, *x = c + a.nmax;
+  const int col_ = blockIdx.x;
+  for (int l = a.top; l > a.bl; --l) {
+    const CLevel<T> &L = a.lv[l];
+    const size_t o = cld(L.vs) * (size_t)col_;
+    const int n = cld(L.n);
+    T *cg = (l == a.top ? a.c_top : cld(L.c)) + o, *bg = (l == a.top ? a.b_top : cld(L.b)) + o;
+    const int cmode = l == a.top ? a.cmode : 0;
+    if (l == a.top) {
+      wg_copy(n, b, bg);
+      // the first sweep's zero phantoms read t at colours not yet swept
+      for (int i = threadIdx.x; i < n; i += kCoarseThreads) t[i] = (T)0;
+    }
+    if (cmode) wg_copy(n, c, cg);
+    else if (a.nu == 0)
+      for (int i = threadIdx.x; i < n; i += kCoarseThreads) c[i] = (T)0;
+    __syncthreads();
+    wg_smooth(L, col_, a.smoother, a.damp, a.nu, cmode, t, b, c);
+    wg_copy(n, cg, c);
+    wg_copy(n, bg, b);
+    if (l - 1 == a.bl) break;
+    const CLevel<T> &C = a.lv[l - 1];
+    const int nc = cld(C.n);
+    const uint8_t *__restrict__ vnclass = cld(C.vnclass);
+    const uint32_t *__restrict__ skip = cld(C.skip);
+    wg_copy(nc, x, (const T *)cld(C.b) + cld(C.vs) * (size_t)col_);
+    __syncthreads();
+    wg_slices(L.PT, col_, 0, cld(L.PT.nslices), b,
+              [&](int r) { return (vnclass[r] >= 2 ? 2 : 0) | (int)(skip[r] & 1u); },
+              [&](int r, T s, int f) {
+                const T base = f & 2 ? (T)0 : x[r];
+                x[r] = f & 1 ? base : base + (T)1 * s;
+              });
+    __syncthreads();
+    wg_copy(nc, b, x);
+    __syncthreads();
+  }
+}
+
+template <typename T>
+__global__ __launch_bounds__(kCoarseThreads) void k_coarse_up(CoarseArgs<T> a) {
+  extern __shared__ double sh[];
+  T *t = (T *)sh, *b = t + a.nmax, *c = b + a.nmax, *x = c + a.nmax;
+  const int col_ = blockIdx.x;
+  const CLevel<T> &B = a.lv[a.bl];
+  wg_copy(cld(B.n), x, (const T *)cld(B.c) + cld(B.vs) * (size_t)col_);
+  for (int l = a.bl + 1; l <= a.top; ++l) {
+    const CLevel<T> &L = a.lv[l];
+    const size_t o = cld(L.vs) * (size_t)col_;
+    const int n = cld(L.n);
+    T *cg = (l == a.top ? a.c_top : cld(L.c)) + o, *bg = (l == a.top ? a.b_top : cld(L.b)) + o;
+    const uint32_t *__restrict__ iskip = cld(L.iskip);
+    wg_copy(n, c, cg);
+    wg_copy(n, b, bg);
+    __syncthreads();
+    wg_slices(L.P, col_, 0, cld(L.P.nslices), x, [&](int r) { return (iskip[r] & 1u) != 0; },
+              [&](int r, T s, bool skip) {
+                const T tv = skip ? (T)0 : a.lmgc_damp * s;
+                t[r] = tv;
+                c[r] += tv;
+              });
+    __syncthreads();
+    wg_slices(L.A, col_, 0, cld(L.A.nslices), t, [](int) { return 0; }, [&](int r, T s, int) { b[r] -= s; });
+    __syncthreads();
+    wg_smooth(L, col_, a.smoother, a.damp, a.nu, 1, t, b, c);
+    wg_copy(n, bg, b);
+    if (l == a.top) wg_copy(n, cg, c);
+    else wg_copy(n, x, c);
+    __syncthreads();
   }
 }
 
@@ -2239,12 +2235,15 @@ PERM_INST(float, float)
 #undef PERM_INST
 
 template <typename T>
-void launch_coarse_cycle(hipStream_t st, const CoarseArgs<T> &args, int base_n) {
-  const size_t shmem = 3 * (size_t)base_n * sizeof(double);
-  k_coarse_cycle<T><<<1, kCoarseThreads, shmem, st>>>(args);
+void launch_coarse(hipStream_t st, const CoarseArgs<T> &args, bool up, int nrhs) {
+  const size_t shmem = (3 * (size_t)args.nmax + args.ncmax) * sizeof(T);
+  const void *k = up ? (const void *)k_coarse_up<T> : (const void *)k_coarse_down<T>;
+  (void)hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kCoarseLds);
+  if (up) k_coarse_up<T><<<nrhs, kCoarseThreads, shmem, st>>>(args);
+  else k_coarse_down<T><<<nrhs, kCoarseThreads, shmem, st>>>(args);
 }
-template void launch_coarse_cycle<double>(hipStream_t, const CoarseArgs<double> &, int);
-template void launch_coarse_cycle<float>(hipStream_t, const CoarseArgs<float> &, int);
+template void launch_coarse<double>(hipStream_t, const CoarseArgs<double> &, bool, int);
+template void launch_coarse<float>(hipStream_t, const CoarseArgs<float> &, bool, int);
 
 // ============================================================ BCGSSolver
 // Right-preconditioned BiCGStab of np/procs/ls.cc:1864-2062 for several
