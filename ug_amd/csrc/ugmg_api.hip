@@ -1179,8 +1179,12 @@ int launch_bcgs_iteration(ugmg_ctx *ctx, int level, bool use_iter, int restart, 
 // 9^3 (187e6) 12.3 / 5.6, 11^3 59 / 13
 constexpr double kBaseDeviceWork = 5.0e7;
 
-// the largest level that k_coarse_down and k_coarse_up take
-constexpr int kCoarseRows = 12288;
+// the largest level that k_coarse_down and k_coarse_up take.  A pass over a
+// level's slabs through one CU overtakes the launches it saves at a few
+// thousand rows: 2D Poisson solve 1756 us with none, 1407 us up to 17^2, 1342
+// us up to 33^2, 1633 us up to 65^2; serving 32.0 ms with none, 29.9 ms up to
+// 9^3, 29.7 ms up to 17^3
+constexpr int kCoarseRows = 1200;
 
 // FULLREFINELEVEL of the levels set up to `level` (SetSurfaceClasses,
 // gm/algebra.cc:2885-2916): the lowest level holding a FINE_GRID_DOF vector
