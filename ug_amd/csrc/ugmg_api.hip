@@ -580,14 +580,43 @@ void smooth_step(ugmg_ctx *ctx, int l, T *t, T *b, T *c, int cmode, T *xout, int
   }
 }
 
+// can a Jacobi step's x = damp D^-1 b be formed by the kernel before it?
+bool fold_jac(const ugmg_ctx *ctx, int nsteps, bool post = false) {
+  return sm_kind(ctx, post) == UGMG_SMOOTH_JAC && nsteps >= 1 && ctx->fuse_steps &&
+         !per_comp(ctx, sm_damp(ctx, post));
+}
+
+// nsteps Jacobi steps (fold_jac): x lies in t and u in turn, the first in t
+// if `ready`; every step but the last forms the next one's
+template <typename T>
+void smooth_jac(ugmg_ctx *ctx, int l, T *t, T *u, T *b, T *c, int cmode, int nsteps, bool ready, bool post) {
+  DevLevel &d = ctx->dev[l];
+  hipStream_t st = ctx->stream;
+  const T damp = (T)sm_damp(ctx, post)[0];
+  const Batch bt = batch(ctx, l);
+  if (!ready) launch_jac<T>(st, d.n, b, d.diag<T>(), d.vclass, damp, t, bt);
+  for (int i = 0; i < nsteps; ++i, std::swap(t, u)) {
+    const int mode = i == 0 && cmode == 0 ? 3 : 2;
+    if (i + 1 < nsteps)
+      launch_spmv_jac<T>(st, d.A.d<T>(), t, b, c, mode, d.diag<T>(), d.vclass, damp, u, d.ntv<T>(), bt);
+    else
+      launch_spmv<T, T, T>(st, d.A.d<T>(), 0, d.A.nslices, t, b, c, mode, d.ntv<T>(), bt);
+  }
+}
+
 // nsteps smoother steps (cmode: correction mode of the first).  On a GS
 // level whose rows are all active, the defect of every step but the last is
 // folded into the next step's colour sweeps.  k0 = 1: the first step's
-// colour-0 sweep has already written t (by the kernel that produced b).
+// colour-0 sweep (Jacobi: its x) is already in t (from the kernel that
+// produced b).
 template <typename T>
 void smooth(ugmg_ctx *ctx, int l, T *t, T *b, T *c, int cmode, int nsteps, int k0 = 0,
             bool post = false) {
   DevLevel &d = ctx->dev[l];
+  if (fold_jac(ctx, nsteps, post)) {
+    smooth_jac<T>(ctx, l, t, d.uv<T>(), b, c, cmode, nsteps, k0 == 1, post);
+    return;
+  }
   if (sm_kind(ctx, post) != UGMG_SMOOTH_GS || !d.all_active || nsteps < 2 || !ctx->fuse_steps ||
       per_comp(ctx, sm_damp(ctx, post))) {
     for (int i = 0; i < nsteps; ++i)
@@ -758,8 +787,9 @@ void lmgc(ugmg_ctx *ctx, int l, T *c, T *b, int cmode, bool c0_done = false) {
   // lmgc below (not the base solve or k_coarse_down) also its first
   // pre-smoothing sweep's colour 0
   const bool to_base = l - 1 == ctx->bl;
+  const bool jac0 = fold_jac(ctx, p.nu1);      // or Jacobi's first x
   const bool pre0 = l - 1 > ctx->bl && !in_coarse<T>(ctx, l - 1) && p.gamma >= 1 &&
-                    fold_colour0(ctx, l - 1, p.nu1);
+                    (jac0 || fold_colour0(ctx, l - 1, p.nu1));
   // onto the base level (scalar) also b in the inverse's column order, into
   // the base level's spare vector u, for the first base iteration.  With
   // several vector types the base solve forms its own per-type norms.
@@ -768,9 +798,9 @@ void lmgc(ugmg_ctx *ctx, int l, T *c, T *b, int cmode, bool c0_done = false) {
                     p.base_iter == UGMG_BASE_EX;
   const int np = launch_restrict<T>(st, d.PT.d<T>(), dc.skip, dc.vnclass, dc.vclass, b, (T)1,
                                     dc.bv<T>(), to_base && !typed ? ctx->base_part : nullptr, d.ntv<T>(), nb,
-                                    d.vs, dc.vs, d.nb, pre0 ? dc.c0 : nullptr, dc.diag<T>(),
+                                    d.vs, dc.vs, d.nb, pre0 && !jac0 ? dc.c0 : nullptr, dc.diag<T>(),
                                     pre0 ? dc.tv<T>() : nullptr, bcol ? ctx->base_cpos : nullptr,
-                                    dc.uv<T>(), dc.dms);
+                                    dc.uv<T>(), dc.dms, jac0 ? (T)sm_damp(ctx, false)[0] : (T)1);
   if (p.gamma <= 0) launch_fill<T>(st, dc.n, dc.cv<T>(), (T)0, batch(ctx, l - 1));
   for (int g = 0; g < p.gamma; ++g) {
     if (to_base) {
@@ -799,6 +829,13 @@ void lmgc(ugmg_ctx *ctx, int l, T *c, T *b, int cmode, bool c0_done = false) {
   }
   if (fold_colour0(ctx, l, p.nu2, true)) {
     post_smooth_folded<T>(ctx, l, t, b, c, p.nu2);
+    return;
+  }
+  if (fold_jac(ctx, p.nu2, true)) {
+    T *u = d.uv<T>();
+    launch_spmv_jac<T>(st, d.A.d<T>(), t, b, (T *)nullptr, 0, d.diag<T>(), d.vclass, (T)sm_damp(ctx, true)[0], u,
+                       d.ntv<T>(), batch(ctx, l));
+    smooth_jac<T>(ctx, l, u, t, b, c, 1, p.nu2, true, true);
     return;
   }
   launch_spmv<T, T, T>(st, d.A.d<T>(), 0, d.A.nslices, t, b, (T *)nullptr, 0, d.ntv<T>(),
@@ -976,8 +1013,12 @@ double smooth_bytes(const ugmg_ctx *ctx, int l, int sv, int cmode, int nsteps, i
   const DevLevel &d = ctx->dev[l];
   double by = 0.0;
   if (sm_kind(ctx, post) == UGMG_SMOOTH_JAC) {
+    // x formed by the kernel before (every step but an unready first one):
+    // b is at hand there
+    const bool fold = fold_jac(ctx, nsteps, post);
     for (int i = 0; i < nsteps; ++i)
-      by += op_bytes(ctx, l, Op::Jac, sv) + d.A.bytes(sv) + vbytes(d, sv) * ((i == 0 && cmode == 0) ? 4.0 : 5.0);
+      by += op_bytes(ctx, l, Op::Jac, sv) - (fold && (i > 0 || k0 == 1) ? vbytes(d, sv) : 0.0) + d.A.bytes(sv) +
+            vbytes(d, sv) * ((i == 0 && cmode == 0) ? 4.0 : 5.0);
     return by;
   }
   if (!d.all_active || nsteps < 2 || !ctx->fuse_steps || per_comp(ctx, sm_damp(ctx, post))) {
@@ -1024,9 +1065,10 @@ double lmgc_bytes(const ugmg_ctx *ctx, int l, int sv, int cmode, bool c0_done) {
   double by = smooth_bytes(ctx, l, sv, cmode, p.nu1, c0_done ? 1 : 0);
   if (p.nu1 == 0 && cmode == 0) by += vbytes(d, sv);
   const bool to_base = l - 1 == ctx->bl;
-  const bool pre0 = l - 1 > ctx->bl && p.gamma >= 1 && fold_colour0(ctx, l - 1, p.nu1);
+  const bool jac0 = fold_jac(ctx, p.nu1);
+  const bool pre0 = l - 1 > ctx->bl && p.gamma >= 1 && (jac0 || fold_colour0(ctx, l - 1, p.nu1));
   by += op_bytes(ctx, l, Op::Restrict, sv);
-  if (pre0) by += dc.n + (double)dc.color_rows[0] * 2.0 * sv;
+  if (pre0 && !jac0) by += dc.n + (double)dc.color_rows[0] * 2.0 * sv;
   if (to_base && ctx->nb == 1 && ctx->base_cpos && !ctx->base.failed && !dc.vt &&
       p.base_iter == UGMG_BASE_EX)
     by += 4.0 * dc.n + (double)ctx->base_ncyc * sv;
@@ -1037,7 +1079,8 @@ double lmgc_bytes(const ugmg_ctx *ctx, int l, int sv, int cmode, bool c0_done) {
   by += op_bytes(ctx, l, Op::Interp, sv);
   if (fold_colour0(ctx, l, p.nu2, true))
     return by + op_bytes(ctx, l, Op::SpmvC0, sv) + smooth_bytes(ctx, l, sv, 1, p.nu2, 1, true);
-  return by + op_bytes(ctx, l, Op::Spmv, sv) + smooth_bytes(ctx, l, sv, 1, p.nu2, 0, true);
+  return by + op_bytes(ctx, l, Op::Spmv, sv) +
+         smooth_bytes(ctx, l, sv, 1, p.nu2, fold_jac(ctx, p.nu2, true) ? 1 : 0, true);
 }
 
 double cycle_bytes(const ugmg_ctx *ctx, int l, int sv) { return lmgc_bytes(ctx, l, sv, 0, false); }

@@ -144,6 +144,11 @@ template <typename TV, typename T>
 void launch_gs_color_fused(hipStream_t st, const DSell<TV> &L, const DSell<TV> &U, int slice0,
                            int nsl, int wmax_l, int wmax_u, T *b, const T *diag, T damp, T *v,
                            T *c, int cmode, bool nt, Batch bt, bool split);
+// y -= A x (mode 2, 3: and c += x, c = x), plus the next Jacobi step's xn =
+// damp y / diag (0 for VCLASS < 3); xn is not x
+template <typename T>
+void launch_spmv_jac(hipStream_t st, const DSell<T> &A, const T *x, T *y, T *c, int mode, const T *diag,
+                     const uint8_t *vclass, T damp, T *xn, bool nt, Batch bt);
 // y -= A x on a GS level's colour-grouped rows, plus u = y / diag on the rows
 // of colour 0 (the next sweep's first colour; scalar, every row active)
 template <typename TV, typename T>
@@ -154,8 +159,9 @@ void launch_gs_defect(hipStream_t st, const DSell<TV> &U, const T *v, T *b, cons
                       T damp, T *c, int cmode, T *xout, bool nt, Batch bt);
 // returns the number of blocks per column (= partial sums per column when
 // part != null; column j's partials start at part + j * return value).
-// With ct (scalar only) also ct_r = bc_r / cdiag_r on the coarse rows whose
-// cc0 flag is set: the coarse GS pre-smoother's colour-0 sweep.  With cpos
+// With ct also ct_r = cdamp bc_r / cdiag_r (0 for VCLASS < 3): on the coarse
+// rows whose cc0 flag is set, the coarse GS pre-smoother's colour-0 sweep
+// (scalar, cdamp 1), or with cc0 null on all, its first Jacobi step.  With cpos
 // (scalar only) also cbc[cpos_r] = bc_r where cpos_r >= 0: b in the base
 // inverse's column order.
 template <typename T>
@@ -163,7 +169,7 @@ int launch_restrict(hipStream_t st, const DSell<T> &PT, const uint32_t *cskip,
                     const uint8_t *cvnclass, const uint8_t *cvclass, const T *bf, T damp, T *bc,
                     double *part, bool nt, int nrhs, size_t vsf, size_t vsc, int b,
                     const uint8_t *cc0 = nullptr, const T *cdiag = nullptr, T *ct = nullptr,
-                    const int *cpos = nullptr, T *cbc = nullptr, size_t cdms = 0);
+                    const int *cpos = nullptr, T *cbc = nullptr, size_t cdms = 0, T cdamp = 1);
 // Element lists of one level on the device (all pointers device memory):
 // nelem elements of nc corners, elem[e*nc + i] = vector of corner i; element
 // matrices (nc b) x (nc b) row-major over corner-major scalar unknowns,

@@ -429,6 +429,38 @@ __global__ __launch_bounds__(kBlock) void k_spmv(DSell<TV> A, int slice0, int ns
   }
 }
 
+// The same (MODE 0, 2, 3) and the next Jacobi step's x from the new y: xn_r =
+// damp y_r / a_rr, 0 for VCLASS < 3 (the values of k_jac; xn is another
+// vector than x, which other rows still read).  A Jacobi step is then one
+// launch and reads y once: k_jac took 1.5 to 4.8 us a step (locally refined
+// elasticity, mixed, 23.5 -> 22.2 ms; 2D Poisson solve 1350 -> 1231 us).
+template <int MW, typename T, int MODE, int NT>
+__global__ __launch_bounds__(kBlock) void k_spmv_jac(DSell<T> A, int nsl, const T *__restrict__ x,
+                                                      T *__restrict__ y, T *__restrict__ c,
+                                                      const T *__restrict__ diag,
+                                                      const uint8_t *__restrict__ vclass, T damp,
+                                                      T *__restrict__ xn, size_t vs) {
+  SLICE_PROLOGUE(A, 0, nsl)
+  const size_t o = (size_t)col_ * vs;
+  x += o;
+  T yr = 0, dr = 1, xr = 0, cr = 0;
+  int act = 0;
+  if (r >= 0) {
+    yr = y[o + r];
+    dr = diag[A.dms * col_ + r];
+    act = vclass[r] >= 3;
+    if (MODE != 0) xr = x[r];
+    if (MODE == 2) cr = c[o + r];
+  }
+  const T sum = sell_dot<MW, NT, T, T, T>(MV(A) + e0 + lane, A.col + e0 + lane, w, x, sdo, A.dtab, rb);
+  if (r < 0) return;
+  const T yn = yr - sum;
+  y[o + r] = yn;
+  if (MODE == 2) c[o + r] = cr + xr;
+  if (MODE == 3) c[o + r] = xr;
+  xn[o + r] = act ? (yn / dr) * damp : (T)0;
+}
+
 // y -= A x over a GS level's colour-grouped rows, and for the rows of colour
 // 0 (slices below ncs0) also the next GS sweep's colour 0, u_r = y_r / a_rr
 // (colour 0 has no lower neighbours; every row active): the separate sweep
@@ -646,7 +678,7 @@ __global__ __launch_bounds__(kBlock) void k_restrict(DSell<T> PT, int nsl,
                                                       const T *__restrict__ cdiag,
                                                       T *__restrict__ ct,
                                                       const int *__restrict__ cpos,
-                                                      T *__restrict__ cbc, size_t cdms) {
+                                                      T *__restrict__ cbc, size_t cdms, T cdamp) {
   __shared__ double red[kBlock / 64];
   SLICE_PROLOGUE_RED(PT, nsl)
   bf += (size_t)col_ * vsf;
@@ -658,9 +690,10 @@ __global__ __launch_bounds__(kBlock) void k_restrict(DSell<T> PT, int nsl,
       const T base = cvnclass[r] >= 2 ? (T)0 : bc[r];
       const T v = (cskip[r] & 1u) ? base : base + damp * sum;
       bc[r] = v;
-      // the coarse pre-smoother's colour-0 sweep: no lower neighbours, so
-      // its value is (b_r - 0) / a_rr
-      if (ct && cc0[r]) ct[(size_t)col_ * vsc + r] = v / cdiag[cdms * col_ + r];
+      // the coarse pre-smoother's colour-0 sweep (no lower neighbours, so its
+      // value is (b_r - 0) / a_rr; cdamp is 1), or Jacobi's first step
+      if (ct && (!cc0 || cc0[r]))
+        ct[(size_t)col_ * vsc + r] = cvclass[r] >= 3 ? (v / cdiag[cdms * col_ + r]) * cdamp : (T)0;
       // b in the base inverse's column order
       if (cpos) {
         const int pj = cpos[r];
@@ -792,6 +825,36 @@ __global__ __launch_bounds__(kBlock) void k_spmv_bk(DSell<TV> A, int slice0, int
       if (MODE == 3) c[o + q] = (TY)x[q];
     }
   }
+}
+
+// the same and the next Jacobi step's x, as k_spmv_jac
+template <int B, typename T, int MODE, int NT>
+__global__ __launch_bounds__(kBlock) void k_spmv_jac_bk(DSell<T> A, int nsl, const T *__restrict__ x,
+                                                         T *__restrict__ y, T *__restrict__ c,
+                                                         const T *__restrict__ diag,
+                                                         const uint8_t *__restrict__ vclass, T damp,
+                                                         T *__restrict__ xn, size_t vs) {
+  SLICE_PROLOGUE(A, 0, nsl)
+  const size_t o = (size_t)col_ * vs;
+  x += o;
+  T sum[B];
+  sell_dot_blk<B, NT, T, T, T>(MV(A) + e0 + lane, A.pst, A.col + e0 + lane, w, x, sdo, A.dtab, rb, sum);
+  if (r < 0) return;
+  const size_t q0 = (size_t)B * r;
+  T m[B * B], yn[B], xv[B] = {};
+#pragma unroll
+  for (int q = 0; q < B * B; ++q) m[q] = diag[A.dms * col_ + B * q0 + q];
+#pragma unroll
+  for (int i = 0; i < B; ++i) {
+    yn[i] = y[o + q0 + i] - sum[i];
+    y[o + q0 + i] = yn[i];
+    if (MODE == 2) c[o + q0 + i] += x[q0 + i];
+    if (MODE == 3) c[o + q0 + i] = x[q0 + i];
+  }
+  const bool act = vclass[r] >= 3;
+  if (act) solve_small<B, T>(m, yn, xv);
+#pragma unroll
+  for (int i = 0; i < B; ++i) xn[o + q0 + i] = act ? xv[i] * damp : (T)0;
 }
 
 template <int B, int NT>
@@ -951,7 +1014,8 @@ __global__ __launch_bounds__(kBlock) void k_restrict_bk(DSell<T> PT, int nsl,
                                                          const T *__restrict__ bf, T damp,
                                                          T *__restrict__ bc,
                                                          double *__restrict__ part, size_t vsf,
-                                                         size_t vsc) {
+                                                         size_t vsc, const T *__restrict__ cdiag,
+                                                         T *__restrict__ ct, size_t cdms, T cdamp) {
   __shared__ double red[B][kBlock / 64];
   SLICE_PROLOGUE_RED(PT, nsl)
   bf += (size_t)col_ * vsf;
@@ -966,6 +1030,7 @@ __global__ __launch_bounds__(kBlock) void k_restrict_bk(DSell<T> PT, int nsl,
     if (r >= 0) {
       const bool zero = cvnclass[r] >= 2;
       const uint32_t sk = cskip[r];
+      T bn[B], xv[B] = {};
 #pragma unroll
       for (int q = 0; q < B; ++q) {
         const size_t k = (size_t)B * r + q;
@@ -973,8 +1038,20 @@ __global__ __launch_bounds__(kBlock) void k_restrict_bk(DSell<T> PT, int nsl,
         const T v = ((sk >> q) & 1u) ? base
                     : MAT           ? (zero ? damp * sum[q] : base + sum[q])
                                     : base + damp * sum[q];
-        bc[k] = v;
+        bc[k] = bn[q] = v;
         if (part && cvclass[r] >= 2) sq[q] = (double)v * (double)v;
+      }
+      // the coarse pre-smoother's first Jacobi step
+      if (ct) {
+        const bool act = cvclass[r] >= 3;
+        if (act) {
+          T m[B * B];
+#pragma unroll
+          for (int q = 0; q < B * B; ++q) m[q] = cdiag[cdms * col_ + (size_t)B * B * r + q];
+          solve_small<B, T>(m, bn, xv);
+        }
+#pragma unroll
+        for (int q = 0; q < B; ++q) ct[(size_t)col_ * vsc + (size_t)B * r + q] = act ? xv[q] * cdamp : (T)0;
       }
     }
   }
@@ -1559,6 +1636,32 @@ template void launch_spmv<double, double, double>(hipStream_t, const DSell<doubl
 template void launch_spmv<float, float, float>(hipStream_t, const DSell<float> &, int, int,
                                                const float *, float *, float *, int, bool, Batch);
 
+template <typename T>
+void launch_spmv_jac(hipStream_t st, const DSell<T> &A, const T *x, T *y, T *c, int mode, const T *diag,
+                     const uint8_t *vclass, T damp, T *xn, bool nt, Batch bt) {
+  if (A.nslices <= 0) return;
+  const dim3 g = slab_grid(A, 0, A.nslices, bt.nrhs), blk(kBlock);
+#define SPMV_JAC(M)                                                                                       \
+  if (bt.b > 1)                                                                                           \
+    BK_DISPATCH(bt.b, NT_DISPATCH(nt, k_spmv_jac_bk<BK, T, M, NTV><<<g, blk, 0, st>>>(                    \
+                                          A, A.nslices, x, y, c, diag, vclass, damp, xn, bt.vs)));        \
+  else                                                                                                    \
+    W_DISPATCH(A.wmax, NT_DISPATCH(nt, k_spmv_jac<MWV, T, M, NTV><<<g, blk, 0, st>>>(                     \
+                                           A, A.nslices, x, y, c, diag, vclass, damp, xn, bt.vs)))
+  if (mode == 0) {
+    SPMV_JAC(0);
+  } else if (mode == 2) {
+    SPMV_JAC(2);
+  } else {
+    SPMV_JAC(3);
+  }
+#undef SPMV_JAC
+}
+template void launch_spmv_jac<double>(hipStream_t, const DSell<double> &, const double *, double *, double *, int,
+                                      const double *, const uint8_t *, double, double *, bool, Batch);
+template void launch_spmv_jac<float>(hipStream_t, const DSell<float> &, const float *, float *, float *, int,
+                                     const float *, const uint8_t *, float, float *, bool, Batch);
+
 template <typename TV, typename T>
 void launch_spmv_c0(hipStream_t st, const DSell<TV> &A, const T *x, T *y, const T *diag, T *u,
                     int ncs0, bool nt, Batch bt) {
@@ -1769,34 +1872,36 @@ int launch_restrict(hipStream_t st, const DSell<T> &PT, const uint32_t *cskip,
                     const uint8_t *cvnclass, const uint8_t *cvclass, const T *bf, T damp, T *bc,
                     double *part, bool nt, int nrhs, size_t vsf, size_t vsc, int b,
                     const uint8_t *cc0, const T *cdiag, T *ct, const int *cpos, T *cbc,
-                    size_t cdms) {
+                    size_t cdms, T cdamp) {
   if (PT.nslices <= 0) return 0;
   const int g = nblk_slices(PT.nslices);
   if (b > 1 && PT.bb > 1) {
     BK_DISPATCH(b, NT_DISPATCH(nt, k_restrict_bk<BK, T, NTV, true><<<grid2(g, nrhs), kBlock, 0, st>>>(
-                                       PT, PT.nslices, cskip, cvnclass, cvclass, bf, damp, bc, part, vsf, vsc)));
+                                       PT, PT.nslices, cskip, cvnclass, cvclass, bf, damp, bc, part, vsf, vsc, cdiag, ct,
+                                       cdms, cdamp)));
     return g;
   }
   if (b > 1) {
     BK_DISPATCH(b, NT_DISPATCH(nt, k_restrict_bk<BK, T, NTV><<<grid2(g, nrhs), kBlock, 0, st>>>(
-                                       PT, PT.nslices, cskip, cvnclass, cvclass, bf, damp, bc, part, vsf, vsc)));
+                                       PT, PT.nslices, cskip, cvnclass, cvclass, bf, damp, bc, part, vsf, vsc, cdiag, ct,
+                                       cdms, cdamp)));
     return g;
   }
   W_DISPATCH(PT.wmax, NT_DISPATCH(nt, k_restrict<MWV, T, NTV><<<grid2(g, nrhs), kBlock, 0, st>>>(
                                           PT, PT.nslices, cskip, cvnclass, cvclass, bf, damp, bc,
-                                          part, vsf, vsc, cc0, cdiag, ct, cpos, cbc, cdms)));
+                                          part, vsf, vsc, cc0, cdiag, ct, cpos, cbc, cdms, cdamp)));
   return g;
 }
 template int launch_restrict<double>(hipStream_t, const DSell<double> &, const uint32_t *,
                                      const uint8_t *, const uint8_t *, const double *, double,
                                      double *, double *, bool, int, size_t, size_t, int,
                                      const uint8_t *, const double *, double *, const int *,
-                                     double *, size_t);
+                                     double *, size_t, double);
 template int launch_restrict<float>(hipStream_t, const DSell<float> &, const uint32_t *,
                                     const uint8_t *, const uint8_t *, const float *, float,
                                     float *, double *, bool, int, size_t, size_t, int,
                                     const uint8_t *, const float *, float *, const int *, float *,
-                                    size_t);
+                                    size_t, float);
 
 // --------------------------------------------------- base solve (GEMV)
 // A quarter of a row of the inverse times b: columns j0 + 256 m (j0 = 64 q +
