@@ -87,6 +87,41 @@ __device__ __forceinline__ TA sell_dot(const TV *__restrict__ v, const int *__re
   return sum;
 }
 
+// the same for NC columns of x, vs apart (columns past nc repeat the last):
+// an entry's value and column are loaded once and its NC gathers are in
+// flight together
+template <int CH, int NT, int NC, typename TV, typename TX, typename TA>
+__device__ __forceinline__ void sell_dot_mc(const TV *__restrict__ v, const int *__restrict__ ci, int w,
+                                            const TX *__restrict__ x, size_t vs, int nc, int sdo,
+                                            const int *__restrict__ dtab, int rb, TA (&sum)[NC]) {
+#pragma unroll
+  for (int q = 0; q < NC; ++q) sum[q] = 0;
+  const int *__restrict__ dt = dtab + (sdo >= 0 ? sdo : 0);
+  for (int k = 0; k < w; k += CH) {
+    TV a[CH];
+    int c[CH];
+#pragma unroll
+    for (int j = 0; j < CH; ++j) {
+      const int kk = (k + j < w) ? k + j : w - 1;
+      a[j] = ld<NT>(v + 64 * kk);
+      if (sdo < 0) c[j] = ld<NT>(ci + 64 * kk);
+    }
+    if (sdo >= 0)
+#pragma unroll
+      for (int j = 0; j < CH; ++j) c[j] = rb + dt[(k + j < w) ? k + j : w - 1];
+    TX xv[NC][CH];
+#pragma unroll
+    for (int q = 0; q < NC; ++q)
+#pragma unroll
+      for (int j = 0; j < CH; ++j) xv[q][j] = x[(size_t)(q < nc ? q : nc - 1) * vs + c[j]];
+#pragma unroll
+    for (int q = 0; q < NC; ++q)
+#pragma unroll
+      for (int j = 0; j < CH; ++j)
+        if (k + j < w) sum[q] += (TA)a[j] * (TA)xv[q][j];
+  }
+}
+
 // b x b blocks: out_i = sum_k sum_j A_k[i][j] x[b col_k + j] over the row's
 // entries in order, entry k's block in b*b planes of pst values.  A row of
 // 15 to 27 blocks is a chain of rounds (columns, then values and gathers),
@@ -722,6 +757,131 @@ __global__ __launch_bounds__(kBlock) void k_interp(DSell<T> P, int nsl,
   const T tv = (fskip[r] & 1u) ? (T)0 : damp * sum;
   t[o + r] = tv;
   if (CADD) c[o + r] += tv;
+}
+
+// ------------------------------------------------- several columns a row
+// The kernels above with kMc columns of a batch per thread, for one matrix
+// and rows of at most 8 entries (one round of loads).  A workgroup per column
+// reads the entries again from L2 for each and has one column's gathers in
+// flight: 2 TB/s on 32 columns of 513^2.  Sums in the same order, column by
+// column.  BiCGStab on 32 columns of 513^2 21.1 -> 17.7 ms.  Wider rows stay
+// with a workgroup per column: kMc columns of 27 gathers do not fit the
+// registers in one round, and their few workgroups wait for latency.
+constexpr int kMc = 4;
+// the thread's columns col_ .. col_ + nc - 1
+#define MC_COLUMNS(nrhs)                  \
+  const int nc = min(kMc, (nrhs) - kMc * col_); \
+  col_ *= kMc;
+
+template <typename T, int NT, int BS>
+__global__ __launch_bounds__(BS) void k_gs_color_mc(DSell<T> L, int slice0, int nsl, int nrhs,
+                                                     const T *__restrict__ b, const T *__restrict__ diag,
+                                                     const uint8_t *__restrict__ vclass, T *__restrict__ v,
+                                                     size_t vs) {
+  SLICE_PROLOGUE_BS(L, slice0, nsl, BS)
+  MC_COLUMNS(nrhs)
+  b += (size_t)col_ * vs;
+  v += (size_t)col_ * vs;
+  T br[kMc] = {}, dr = 1, sum[kMc];
+  int act = 0;
+  if (r >= 0) {
+#pragma unroll
+    for (int q = 0; q < kMc; ++q) br[q] = b[(size_t)(q < nc ? q : nc - 1) * vs + r];
+    dr = diag[r];
+    act = vclass[r] >= 3;
+  }
+  sell_dot_mc<8, NT, kMc, T, T, T>(L.val + e0 + lane, L.col + e0 + lane, w, v, vs, nc, sdo, L.dtab, rb, sum);
+  if (r < 0) return;
+#pragma unroll
+  for (int q = 0; q < kMc; ++q)
+    if (q < nc) v[(size_t)q * vs + r] = act ? (br[q] - sum[q]) / dr : (T)0;
+}
+
+template <typename T, int CMODE, int NT>
+__global__ __launch_bounds__(kBlock) void k_gs_defect_mc(DSell<T> U, int nsl, int nrhs, const T *__restrict__ v,
+                                                          T *__restrict__ b, const uint8_t *__restrict__ vclass,
+                                                          T damp, T *__restrict__ c, size_t vs) {
+  SLICE_PROLOGUE_MAP(U, 0, nsl, true)
+  MC_COLUMNS(nrhs)
+  v += (size_t)col_ * vs;
+  b += (size_t)col_ * vs;
+  c += (size_t)col_ * vs;
+  T br[kMc] = {}, vr[kMc] = {}, cr[kMc] = {}, sum[kMc];
+  int act = 0;
+  if (r >= 0) {
+#pragma unroll
+    for (int q = 0; q < kMc; ++q) {
+      const size_t o = (size_t)(q < nc ? q : nc - 1) * vs + r;
+      br[q] = b[o];
+      vr[q] = v[o];
+      if (CMODE == 1) cr[q] = c[o];
+    }
+    act = vclass[r] >= 3;
+  }
+  sell_dot_mc<8, NT, kMc, T, T, T>(U.val + e0 + lane, U.col + e0 + lane, w, v, vs, nc, sdo, U.dtab, rb, sum);
+  if (r < 0) return;
+#pragma unroll
+  for (int q = 0; q < kMc; ++q)
+    if (q < nc) {
+      const size_t o = (size_t)q * vs + r;
+      b[o] = act ? br[q] - damp * (br[q] + sum[q]) : br[q] - damp * sum[q];
+      c[o] = CMODE == 0 ? damp * vr[q] : fma(damp, vr[q], cr[q]);
+    }
+}
+
+template <typename T, int NT>
+__global__ __launch_bounds__(kBlock) void k_spmv_c0_mc(DSell<T> A, int nsl, int nrhs, const T *__restrict__ x,
+                                                        T *__restrict__ y, const T *__restrict__ diag,
+                                                        T *__restrict__ u, int ncs0, size_t vs) {
+  SLICE_PROLOGUE(A, 0, nsl)
+  MC_COLUMNS(nrhs)
+  x += (size_t)col_ * vs;
+  y += (size_t)col_ * vs;
+  u += (size_t)col_ * vs;
+  T yr[kMc] = {}, dr = 1, sum[kMc];
+  if (r >= 0) {
+#pragma unroll
+    for (int q = 0; q < kMc; ++q) yr[q] = y[(size_t)(q < nc ? q : nc - 1) * vs + r];
+    if (s < ncs0) dr = diag[r];
+  }
+  sell_dot_mc<8, NT, kMc, T, T, T>(A.val + e0 + lane, A.col + e0 + lane, w, x, vs, nc, sdo, A.dtab, rb, sum);
+  if (r < 0) return;
+#pragma unroll
+  for (int q = 0; q < kMc; ++q)
+    if (q < nc) {
+      const T yn = yr[q] - sum[q];
+      y[(size_t)q * vs + r] = yn;
+      if (s < ncs0) u[(size_t)q * vs + r] = yn / dr;
+    }
+}
+
+template <typename T, int CADD, int NT>
+__global__ __launch_bounds__(kBlock) void k_interp_mc(DSell<T> P, int nsl, int nrhs,
+                                                       const uint32_t *__restrict__ fskip,
+                                                       const T *__restrict__ cc, T damp, T *__restrict__ t,
+                                                       T *__restrict__ c, size_t vsf, size_t vsc) {
+  SLICE_PROLOGUE_MAP(P, 0, nsl, true)
+  MC_COLUMNS(nrhs)
+  cc += (size_t)col_ * vsc;
+  t += (size_t)col_ * vsf;
+  if (CADD) c += (size_t)col_ * vsf;
+  T cr[kMc] = {}, sum[kMc];
+  bool skip = false;
+  if (r >= 0) {
+    skip = fskip[r] & 1u;
+    if (CADD)
+#pragma unroll
+      for (int q = 0; q < kMc; ++q) cr[q] = c[(size_t)(q < nc ? q : nc - 1) * vsf + r];
+  }
+  sell_dot_mc<4, NT, kMc, T, T, T>(P.val + e0 + lane, P.col + e0 + lane, w, cc, vsc, nc, sdo, P.dtab, rb, sum);
+  if (r < 0) return;
+#pragma unroll
+  for (int q = 0; q < kMc; ++q)
+    if (q < nc) {
+      const T tv = skip ? (T)0 : damp * sum[q];
+      t[(size_t)q * vsf + r] = tv;
+      if (CADD) c[(size_t)q * vsf + r] = cr[q] + tv;
+    }
 }
 
 // -------------------------------------------------------------- reductions
@@ -1609,6 +1769,13 @@ static dim3 slab_grid(const DSell<TV> &S, int slice0, int nsl, int nrhs) {
     }                        \
   } while (0)
 
+// may a batched launch over S take kMc columns a thread?
+template <typename TV>
+static bool mc_columns(const DSell<TV> &S, int wmax, int nrhs) {
+  return nrhs >= kMc && wmax <= 8 && S.mst == 0 && S.dms == 0;
+}
+static int mc_groups(int nrhs) { return (nrhs + kMc - 1) / kMc; }
+
 template <typename TV, typename TX, typename TY>
 void launch_spmv(hipStream_t st, const DSell<TV> &A, int slice0, int nsl, const TX *x, TY *y,
                  TY *c, int mode, bool nt, Batch bt) {
@@ -1666,6 +1833,11 @@ template <typename TV, typename T>
 void launch_spmv_c0(hipStream_t st, const DSell<TV> &A, const T *x, T *y, const T *diag, T *u,
                     int ncs0, bool nt, Batch bt) {
   if (A.nslices <= 0) return;
+  if (mc_columns(A, A.wmax, bt.nrhs)) {
+    NT_DISPATCH(nt, k_spmv_c0_mc<T, NTV><<<slab_grid(A, 0, A.nslices, mc_groups(bt.nrhs)), kBlock, 0, st>>>(
+                        A, A.nslices, bt.nrhs, x, y, diag, u, ncs0, bt.vs));
+    return;
+  }
   const dim3 g = slab_grid(A, 0, A.nslices, bt.nrhs);
   W_DISPATCH(A.wmax, NT_DISPATCH(nt, k_spmv_c0<MWV, TV, T, NTV><<<g, kBlock, 0, st>>>(
                                          A, A.nslices, x, y, diag, u, ncs0, bt.vs)));
@@ -1737,6 +1909,13 @@ void launch_gs_color(hipStream_t st, const DSell<TV> &L, int slice0, int nsl, in
   if (bt.b > 1) {
     BK_DISPATCH(bt.b, GSB_DISPATCH(nsl, NT_DISPATCH(nt, k_gs_color_bk<BK, TV, T, NTV, BSV><<<g, BSV, 0, st>>>(
                                                             L, slice0, nsl, b, diag, vclass, v, bt.vs))));
+    return;
+  }
+  if (mc_columns(L, wmax, bt.nrhs)) {
+    const int nrhs = bt.nrhs;
+    bt.nrhs = mc_groups(nrhs);     // (the grid of GSB_DISPATCH)
+    GSB_DISPATCH(nsl, NT_DISPATCH(nt, k_gs_color_mc<T, NTV, BSV><<<g, BSV, 0, st>>>(L, slice0, nsl, nrhs, b, diag, vclass,
+                                                                                   v, bt.vs)));
     return;
   }
   if constexpr (!std::is_same_v<T, double>) {
@@ -1850,6 +2029,14 @@ void launch_gs_defect(hipStream_t st, const DSell<TV> &U, const T *v, T *b, cons
                         U, U.nslices, v, b, vclass, damp, c, xout, bt.vs);
                 else k_gs_defect_bk<BK, TV, T, 1, NTV><<<g, kBlock, 0, st>>>(
                         U, U.nslices, v, b, vclass, damp, c, xout, bt.vs)));
+    return;
+  }
+  if (mc_columns(U, U.wmax, bt.nrhs) && c && !xout) {
+    const dim3 gm = slab_grid(U, 0, U.nslices, mc_groups(bt.nrhs));
+    NT_DISPATCH(nt, if (cmode == 0) k_gs_defect_mc<T, 0, NTV><<<gm, kBlock, 0, st>>>(
+                        U, U.nslices, bt.nrhs, v, b, vclass, damp, c, bt.vs);
+                else k_gs_defect_mc<T, 1, NTV><<<gm, kBlock, 0, st>>>(
+                        U, U.nslices, bt.nrhs, v, b, vclass, damp, c, bt.vs));
     return;
   }
   // chunks of 8 entries: the upper widths of the colours run from the whole
@@ -2154,6 +2341,12 @@ void launch_interp(hipStream_t st, const DSell<T> &P, const uint32_t *fskip, con
                                                                                        damp, t, c, vsf, vsc);
                                else k_interp_bk<BK, T, 0, NTV><<<g, kBlock, 0, st>>>(P, P.nslices, fskip, cc,
                                                                                     damp, t, c, vsf, vsc)));
+    return;
+  }
+  if (mc_columns(P, P.wmax, nrhs)) {
+    const dim3 gm = grid2(nblk_slices(P.nslices), mc_groups(nrhs));
+    NT_DISPATCH(nt, if (c) k_interp_mc<T, 1, NTV><<<gm, kBlock, 0, st>>>(P, P.nslices, nrhs, fskip, cc, damp, t, c, vsf, vsc);
+                else k_interp_mc<T, 0, NTV><<<gm, kBlock, 0, st>>>(P, P.nslices, nrhs, fskip, cc, damp, t, c, vsf, vsc));
     return;
   }
   // interpolation rows hold 1, 2, 4 or 8 coarse corners: chunks of 4
@@ -2570,6 +2763,74 @@ __global__ __launch_bounds__(kBlock) void k_bcgs_spmv(DSell<double> A, int nsl,
   }
 }
 
+// the same with kMc columns a thread (k_gs_color_mc)
+template <typename TQ, int NT>
+__global__ __launch_bounds__(kBlock) void k_bcgs_spmv_mc(DSell<double> A, int nsl, int nrhs,
+                                                          const TQ *__restrict__ q, double *__restrict__ y,
+                                                          const double *__restrict__ z,
+                                                          const uint8_t *__restrict__ vclass,
+                                                          double *__restrict__ part, int yy, int skip_half,
+                                                          const BcgsState *__restrict__ st, size_t vs) {
+  __shared__ double red[kMc][2][kBlock / 64];
+  SLICE_PROLOGUE_RED(A, nsl)
+  MC_COLUMNS(nrhs)
+  bool on[kMc], any = false;
+#pragma unroll
+  for (int k = 0; k < kMc; ++k) {
+    on[k] = k < nc && st[col_ + min(k, nc - 1)].active && !(skip_half && st[col_ + min(k, nc - 1)].half);
+    any |= on[k];
+  }
+  if (!any) return;   // uniform per block
+  const size_t o = (size_t)col_ * vs;
+  double yz[kMc] = {}, y2[kMc] = {};
+  if (sok) {
+    double sum[kMc], zr[kMc] = {};
+    if (r >= 0)
+#pragma unroll
+      for (int k = 0; k < kMc; ++k) zr[k] = z[o + (size_t)min(k, nc - 1) * vs + r];
+    sell_dot_mc<8, NT, kMc, double, TQ, double>(A.val + e0 + lane, A.col + e0 + lane, w, q + o, vs, nc, sdo, A.dtab,
+                                                rb, sum);
+    if (r >= 0) {
+      const bool in = vclass[r] >= 2;
+#pragma unroll
+      for (int k = 0; k < kMc; ++k)
+        if (on[k]) {
+          y[o + (size_t)k * vs + r] = sum[k];
+          if (in) {
+            yz[k] = sum[k] * zr[k];
+            y2[k] = sum[k] * sum[k];
+          }
+        }
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < kMc; ++k) {
+    for (int off = 32; off > 0; off >>= 1) {
+      yz[k] += __shfl_down(yz[k], off, 64);
+      y2[k] += __shfl_down(y2[k], off, 64);
+    }
+    if (lane == 0) {
+      red[k][0][threadIdx.x >> 6] = yz[k];
+      red[k][1][threadIdx.x >> 6] = y2[k];
+    }
+  }
+  __syncthreads();
+  const int k = threadIdx.x;
+  if (k >= nc || !st[col_ + k].active || (skip_half && st[col_ + k].half)) return;
+  double a = 0.0, b2 = 0.0;
+  for (int i = 0; i < kBlock / 64; ++i) {
+    a += red[k][0][i];
+    b2 += red[k][1][i];
+  }
+  double *pp = part + (size_t)((col_ + k) * 2) * gridDim.x;
+  if (yy) {
+    pp[sb_] = b2;
+    pp[gridDim.x + sb_] = a;
+  } else {
+    pp[sb_] = a;
+  }
+}
+
 template <typename TQ>
 void launch_bcgs_spmv(hipStream_t st, const DSell<double> &A, const TQ *q, double *y,
                       const double *z, const uint8_t *vclass, double *part, int yy, int skip_half, const BcgsState *s, bool nt, Batch bt) {
@@ -2577,6 +2838,11 @@ void launch_bcgs_spmv(hipStream_t st, const DSell<double> &A, const TQ *q, doubl
   const dim3 g = grid2(nblk_slices(A.nslices), bt.nrhs);
   DSell<double> Ap = A;
   Ap.ncb = 0;   // its partial sums are strided by the grid: the plain map
+  if (mc_columns(A, A.wmax, bt.nrhs)) {
+    NT_DISPATCH(nt, k_bcgs_spmv_mc<TQ, NTV><<<grid2(nblk_slices(A.nslices), mc_groups(bt.nrhs)), kBlock, 0, st>>>(
+                        Ap, A.nslices, bt.nrhs, q, y, z, vclass, part, yy, skip_half, s, bt.vs));
+    return;
+  }
   W_DISPATCH(A.wmax, NT_DISPATCH(nt, k_bcgs_spmv<MWV, TQ, NTV><<<g, kBlock, 0, st>>>(
                                          Ap, A.nslices, q, y, z, vclass, part, yy, skip_half, s,
                                          bt.vs)));
