@@ -69,3 +69,25 @@ def test_coarse_levels_are_bitwise_the_separate_launches(k, monkeypatch):
     for rows in (None, P.levels[-2].n, P.levels[-2].n - 1):
         got = _cycle(P, monkeypatch, rows, **kw)
         assert np.array_equal(got[0], want[0]) and np.array_equal(got[1], want[1]), rows
+
+
+@pytest.mark.parametrize("smoother,damp", [(ugmg.SMOOTH_JAC, 0.8), (ugmg.SMOOTH_GS, 1.0)])
+def test_surface_solve_is_bitwise_the_separate_launches(smoother, damp, monkeypatch):
+    """Every level's correction is there after a cycle: the surface solve adds
+    them into x level by level."""
+    P = problems.p1_local(4, 2)
+    fs = problems.surface_rhs(P, 1, 4)
+    out = []
+    for rows in (0, 12288):
+        monkeypatch.setenv("UGMG_FUSE_ROWS", str(rows))
+        ctx = ugmg.Context(0)
+        ctx.set_hierarchy(P)
+        ctx.set_params(nu1=2, nu2=2, gamma=1, baselevel=1, smoother=smoother, damp=damp, base_abslimit=1e-300,
+                       base_maxiter=1)
+        ctx.preprocess()
+        out.append(ctx.solve_surface_host(P.top, fs, red=1e-8, maxiter=30))
+        ctx.close()
+    (x0, b0, r0, _), (x1, b1, r1, _) = out
+    assert r0.number_of_linear_iterations == r1.number_of_linear_iterations
+    for l in range(1, P.top + 1):
+        assert np.array_equal(x0[l], x1[l]) and np.array_equal(b0[l], b1[l]), l

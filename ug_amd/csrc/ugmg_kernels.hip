@@ -1698,8 +1698,8 @@ __global__ __launch_bounds__(kCoarseThreads) void k_coarse_up(CoarseArgs<T> a) {
     __syncthreads();
     wg_smooth(L, col_, a.smoother, a.damp, a.nu, 1, t, b, c);
     wg_copy(n, bg, b);
-    if (l == a.top) wg_copy(n, cg, c);
-    else wg_copy(n, x, c);
+    wg_copy(n, cg, c);                   // (a solve on the surface adds every level's correction)
+    if (l < a.top) wg_copy(n, x, c);
     __syncthreads();
   }
 }
