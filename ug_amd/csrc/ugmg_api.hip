@@ -233,6 +233,12 @@ struct ugmg_ctx {
   static constexpr int kMaxGraphs = 65;
   hipGraphExec_t gexec[kMaxGraphs] = {};
   int gkind = -1, glevel = -1;
+  // ugmg_iter's cycle on a level's own vectors: its graph, and the calls it
+  // has served (the first one records nothing)
+  struct IterGraph {
+    hipGraphExec_t g = nullptr;
+    int level = -1, nb = 0, calls = 0;
+  } ig;
   const void *gx = nullptr, *gb = nullptr;
   // members: `members` matrices of one pattern, one per column of the
   // level vectors (batched launches read column j's values, diagonal
@@ -465,6 +471,8 @@ void drop_graph(ugmg_ctx *ctx) {
       g = nullptr;
     }
   ctx->sgkind = -1;
+  if (ctx->ig.g) hipGraphExecDestroy(ctx->ig.g);
+  ctx->ig = ugmg_ctx::IterGraph();
   drop_bcgs_graphs(ctx);
 }
 
@@ -1095,6 +1103,56 @@ double iteration_bytes(const ugmg_ctx *ctx, int l, int cycles) {
   for (int j = 0; j < cycles; ++j) by += lmgc_bytes(ctx, l, 4, j == 0 ? 0 : 1, false);
   return by + d.A.bytes(8) + (double)d.n * d.nb * (4.0 + 4.0 + 16.0 + 16.0 + 4.0) + d.n;
 }
+
+// The cycle of ugmg_iter (inner_cycles of them in FP32) on the level's own
+// vectors.  From the second call with the same level and columns on it is
+// replayed from a graph: a launch per operation takes the host 2.3 to 3 us,
+// as long as small levels take the device or longer (8 columns of 33^3: 307
+// us a call, 187 us replayed).  A stream that is being captured gets the
+// launches.
+int own_cycle(ugmg_ctx *ctx, int level) {
+  DevLevel &d = ctx->dev[level];
+  auto enqueue = [&] {
+    if (ctx->p.precision == UGMG_MIXED) {
+      const int k = std::max(1, ctx->p.inner_cycles);
+      for (int j = 0; j < k; ++j) lmgc<float>(ctx, level, d.c32, d.b32, j == 0 ? 0 : 1);
+    } else {
+      lmgc<double>(ctx, level, d.c, d.b, 0);
+    }
+  };
+  auto &ig = ctx->ig;
+  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+  if (can_capture(ctx)) HIPCHK(hipStreamIsCapturing(ctx->stream, &cs));
+  if (ig.level != level || ig.nb != ctx->nb) {
+    if (ig.g) hipGraphExecDestroy(ig.g);
+    ig = ugmg_ctx::IterGraph();
+    ig.level = level;
+    ig.nb = ctx->nb;
+  }
+  if (!can_capture(ctx) || cs != hipStreamCaptureStatusNone || ig.calls++ == 0) {
+    enqueue();
+    HIPCHK(hipGetLastError());
+    return 0;
+  }
+  if (!ig.g) {
+    hipGraph_t g = nullptr;
+    HIPCHK(hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeThreadLocal));
+    enqueue();
+    HIPCHK(hipStreamEndCapture(ctx->stream, &g));
+    hipError_t e = hipGraphInstantiate(&ig.g, g, nullptr, nullptr, 0);
+    hipGraphDestroy(g);
+    if (e != hipSuccess) {
+      ig.g = nullptr;
+      return fail(ctx, UGMG_E_HIP, std::string("hipGraphInstantiate: ") + hipGetErrorString(e));
+    }
+  }
+  HIPCHK(hipGraphLaunch(ig.g, ctx->stream));
+  return 0;
+}
+
+// levels kept in list order: up to this many values the two copies to and
+// from the level's own vectors are cheaper than the launches
+constexpr size_t kOwnCycleValues = 65536;
 
 // ------------------------------------------------------------ BCGSSolver
 // Work of BCGSSolver (np/procs/ls.cc:1864-2062) on nb columns of level
@@ -2558,8 +2616,7 @@ int ugmg_iter(ugmg_ctx *ctx, int level, double *c, double *b) {
   DevLevel &d = ctx->dev[level];
   if (ctx->p.precision == UGMG_MIXED) {
     to_dev<float, double>(ctx, level, b, d.vs, d.b32);
-    const int k = std::max(1, ctx->p.inner_cycles);
-    for (int j = 0; j < k; ++j) lmgc<float>(ctx, level, d.c32, d.b32, j == 0 ? 0 : 1);
+    if ((rc = own_cycle(ctx, level))) return rc;
     if (!d.perm) {
       launch_convert<double, float>(ctx->stream, d.n * d.nb, d.c32, c, 1, d.vs, d.vs);
       launch_spmv<double, double, double>(ctx->stream, d.A.d64(), 0, d.A.nslices, c, b, nullptr, 0, d.nt, B1(d));
@@ -2570,11 +2627,11 @@ int ugmg_iter(ugmg_ctx *ctx, int level, double *c, double *b) {
       to_user<double, double>(ctx, level, d.c, c, d.vs);
       to_user<double, double>(ctx, level, d.b, b, d.vs);
     }
-  } else if (!d.perm) {
+  } else if (!d.perm && (!can_capture(ctx) || (size_t)d.n * d.nb > kOwnCycleValues)) {
     lmgc<double>(ctx, level, c, b, 0);
   } else {
     to_dev<double, double>(ctx, level, b, d.vs, d.b);
-    lmgc<double>(ctx, level, d.c, d.b, 0);
+    if ((rc = own_cycle(ctx, level))) return rc;
     to_user<double, double>(ctx, level, d.c, c, d.vs);
     to_user<double, double>(ctx, level, d.b, b, d.vs);
   }
@@ -3118,18 +3175,18 @@ int ugmg_iter_batch(ugmg_ctx *ctx, int level, int nrhs, double *c, double *b, in
   const Batch bt = batch(ctx, level);
   if (ctx->p.precision == UGMG_MIXED) {
     to_dev<float, double>(ctx, level, b, ld, d.b32, nrhs);
-    const int k = std::max(1, ctx->p.inner_cycles);
-    for (int j = 0; j < k; ++j) lmgc<float>(ctx, level, d.c32, d.b32, j == 0 ? 0 : 1);
+    rc = own_cycle(ctx, level);
     launch_convert<double, float>(st, d.n * d.nb, d.c32, d.c, nrhs, d.vs, d.vs);
     to_dev<double, double>(ctx, level, b, ld, d.b, nrhs);
     launch_spmv<double, double, double>(st, d.A.d64(), 0, d.A.nslices, d.c, d.b, nullptr, 0, d.nt, bt);
   } else {
     to_dev<double, double>(ctx, level, b, ld, d.b, nrhs);
-    lmgc<double>(ctx, level, d.c, d.b, 0);
+    rc = own_cycle(ctx, level);
   }
   to_user<double, double>(ctx, level, d.c, c, ld, nrhs);
   to_user<double, double>(ctx, level, d.b, b, ld, nrhs);
   ctx->nb = 1;
+  if (rc) return rc;
   HIPCHK(hipGetLastError());
   return UGMG_OK;
 }
