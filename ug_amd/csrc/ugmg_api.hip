@@ -283,7 +283,7 @@ struct ugmg_ctx {
   // batched launches: level vectors hold nrhs_cap columns; nb = columns of
   // the work being enqueued
   int nrhs_cap = 1, nb = 1;
-  bool fuse_steps = true;   // fold GS defects into the next sweep (UGMG_GS_FUSE=0: off)
+  bool fuse_steps = true;   // fold GS defects into the next sweep, Jacobi x into the kernel before (UGMG_GS_FUSE=0: off)
   // folded sweeps with the upper and lower row products on two wavefronts
   // per slice (UGMG_GS_SPLIT=0: one wavefront per slice)
   bool gs_split = true;
