@@ -1640,11 +1640,11 @@ __global__ __launch_bounds__(kCoarseThreads) void k_coarse_down(CoarseArgs<T> a)
     const int n = cld(L.n);
     T *cg = (l == a.top ? a.c_top : cld(L.c)) + o, *bg = (l == a.top ? a.b_top : cld(L.b)) + o;
     const int cmode = l == a.top ? a.cmode : 0;
-    if (l == a.top) {
-      wg_copy(n, b, bg);
-      // the first sweep's zero phantoms read t at colours not yet swept
+    if (l == a.top) wg_copy(n, b, bg);
+    // the first colour sweep's zero phantoms read t at colours not yet swept,
+    // up to this level's n (a lower level may have more vectors than the top)
+    if (a.smoother == 1)
       for (int i = threadIdx.x; i < n; i += kCoarseThreads) t[i] = (T)0;
-    }
     if (cmode) wg_copy(n, c, cg);
     else if (a.nu == 0)
       for (int i = threadIdx.x; i < n; i += kCoarseThreads) c[i] = (T)0;
