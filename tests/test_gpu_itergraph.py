@@ -36,16 +36,17 @@ def test_iter_calls(kw):
     for nu in (1, 2):
         if nu == 2:
             params(2)
-        for k, (level, cols) in enumerate([(4, 1), (4, 1), (4, 1), (4, 3), (4, 3), (3, 1), (3, 1), (4, 1), (4, 1)]):
+        for k, (level, cols) in enumerate([(4, 1), (4, 1), (4, 1), (4, 3), (4, 3), (3, 1), (3, 1), (4, 1), (4, 1),
+                                           (4, 0), (4, 1), (4, 0), (4, 0)]):     # 0: a batch of one
             lv = P.levels[level]
-            f = np.random.default_rng(100 * nu + k).uniform(-1.0, 1.0, (cols, lv.n))
+            f = np.random.default_rng(100 * nu + k).uniform(-1.0, 1.0, (max(cols, 1), lv.n))
             f[:, lv.skip & 1 == 1] = 0.0
             out = []
             for ctx in ctxs:
                 b = torch.from_numpy(f).cuda()
                 c = torch.zeros_like(b)
                 torch.cuda.synchronize()
-                if cols > 1:
+                if cols != 1:
                     ctx.iter_batch(level, c, b)
                 else:
                     ctx.iter(level, c[0], b[0])
@@ -55,3 +56,37 @@ def test_iter_calls(kw):
             assert np.array_equal(out[0][0], out[1][0]) and np.array_equal(out[0][1], out[1][1]), (nu, k)
     for ctx in ctxs:
         ctx.close()
+
+
+@pytest.mark.parametrize("kw", [
+    dict(smoother=ugmg.SMOOTH_JAC, damp=0.8), dict(smoother=ugmg.SMOOTH_JAC, damp=0.8, nu1=2, nu2=2), dict(),
+    dict(precision=ugmg.MIXED)])
+def test_local_levels(kw):
+    """A cycle on a local level restricts onto the defect that the level below
+    holds outside the refined part; a cycle on the level below's list-order
+    FP64 vectors before it leaves that alone."""
+    P = problems.p1_local(4, 2)
+    assert any(np.any(lv.vnclass < 2) for lv in P.levels[3:-1])
+    out = []
+    for use in (0, 1):
+        ctx = ugmg.Context(0)
+        ctx.set_stream(torch.cuda.Stream())
+        ctx.set_hierarchy(P)
+        ctx.set_params(**{**dict(nu1=1, nu2=1, gamma=1, baselevel=1, smoother=ugmg.SMOOTH_GS, damp=1.0,
+                                 base_abslimit=1e-300, base_maxiter=1, use_graph=use), **kw})
+        ctx.preprocess()
+        got = []
+        for k in range(3):
+            for level in range(2, P.top + 1):
+                lv = P.levels[level]
+                b = torch.from_numpy(np.random.default_rng(10 * k + level).uniform(-1.0, 1.0, lv.n)).cuda()
+                c = torch.zeros_like(b)
+                torch.cuda.synchronize()
+                ctx.iter(level, c, b)
+                ctx.sync()
+                got += [c.cpu().numpy(), b.cpu().numpy()]
+        ctx.close()
+        out.append(got)
+    assert all(np.any(v) for v in out[0])
+    for k, (a, b) in enumerate(zip(*out)):
+        assert np.array_equal(a, b), k

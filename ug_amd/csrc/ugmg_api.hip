@@ -233,12 +233,18 @@ struct ugmg_ctx {
   static constexpr int kMaxGraphs = 65;
   hipGraphExec_t gexec[kMaxGraphs] = {};
   int gkind = -1, glevel = -1;
-  // ugmg_iter's cycle on a level's own vectors: its graph, and the calls it
-  // has served (the first one records nothing)
+  // the cycle of ugmg_iter and ugmg_iter_batch on a level and vectors of the
+  // context (c; null: FP32): its graph, and the calls it has served (the
+  // first one records nothing)
   struct IterGraph {
     hipGraphExec_t g = nullptr;
     int level = -1, nb = 0, calls = 0;
+    const double *c = nullptr;
   } ig;
+  // ugmg_iter's on levels in list order, where launches work on the caller's
+  // vectors: not the level's own, whose b a restriction adds to
+  double *own_c = nullptr, *own_b = nullptr;
+  size_t own_n = 0;
   const void *gx = nullptr, *gb = nullptr;
   // members: `members` matrices of one pattern, one per column of the
   // level vectors (batched launches read column j's values, diagonal
@@ -447,6 +453,8 @@ void free_device(ugmg_ctx *ctx) {
   ctx->base_ncyc = 0;
   ctx->base_nact = 0;
   ctx->base_cpos = nullptr;
+  ctx->own_c = ctx->own_b = nullptr;
+  ctx->own_n = 0;
   ctx->clev64 = nullptr;
   ctx->clev32 = nullptr;
   ctx->fuse_top[0] = ctx->fuse_top[1] = -1;
@@ -1104,32 +1112,42 @@ double iteration_bytes(const ugmg_ctx *ctx, int l, int cycles) {
   return by + d.A.bytes(8) + (double)d.n * d.nb * (4.0 + 4.0 + 16.0 + 16.0 + 4.0) + d.n;
 }
 
-// The cycle of ugmg_iter (inner_cycles of them in FP32) on the level's own
-// vectors.  From the second call with the same level and columns on it is
-// replayed from a graph: a launch per operation takes the host 2.3 to 3 us,
-// as long as small levels take the device or longer (8 columns of 33^3: 307
-// us a call, 187 us replayed).  A stream that is being captured gets the
-// launches.
-int own_cycle(ugmg_ctx *ctx, int level) {
+// Is this call's cycle to be replayed from a graph?  From the second call
+// with the same level, columns and c (own_cycle's) on: a launch per operation takes the
+// host 2.3 to 3 us, as long as small levels take the device or longer (8
+// columns of 33^3: 307 us a call, 187 us replayed).  A stream that is being
+// captured gets the launches.
+int replayed(ugmg_ctx *ctx, int level, const double *c, bool &yes) {
+  yes = false;
+  if (!can_capture(ctx)) return 0;
+  auto &ig = ctx->ig;
+  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+  HIPCHK(hipStreamIsCapturing(ctx->stream, &cs));
+  if (ig.level != level || ig.nb != ctx->nb || ig.c != c) {
+    if (ig.g) hipGraphExecDestroy(ig.g);
+    ig = ugmg_ctx::IterGraph();
+    ig.level = level;
+    ig.nb = ctx->nb;
+    ig.c = c;
+  }
+  yes = cs == hipStreamCaptureStatusNone && ig.calls++ > 0;
+  return 0;
+}
+
+// The cycle of ugmg_iter on c and b, vectors of the context, or (mixed, both
+// null) inner_cycles of them on the level's FP32 vectors
+int own_cycle(ugmg_ctx *ctx, int level, double *c, double *b, bool replay) {
   DevLevel &d = ctx->dev[level];
   auto enqueue = [&] {
     if (ctx->p.precision == UGMG_MIXED) {
       const int k = std::max(1, ctx->p.inner_cycles);
       for (int j = 0; j < k; ++j) lmgc<float>(ctx, level, d.c32, d.b32, j == 0 ? 0 : 1);
     } else {
-      lmgc<double>(ctx, level, d.c, d.b, 0);
+      lmgc<double>(ctx, level, c, b, 0);
     }
   };
   auto &ig = ctx->ig;
-  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-  if (can_capture(ctx)) HIPCHK(hipStreamIsCapturing(ctx->stream, &cs));
-  if (ig.level != level || ig.nb != ctx->nb) {
-    if (ig.g) hipGraphExecDestroy(ig.g);
-    ig = ugmg_ctx::IterGraph();
-    ig.level = level;
-    ig.nb = ctx->nb;
-  }
-  if (!can_capture(ctx) || cs != hipStreamCaptureStatusNone || ig.calls++ == 0) {
+  if (!replay) {
     enqueue();
     HIPCHK(hipGetLastError());
     return 0;
@@ -1150,9 +1168,22 @@ int own_cycle(ugmg_ctx *ctx, int level) {
   return 0;
 }
 
-// levels kept in list order: up to this many values the two copies to and
-// from the level's own vectors are cheaper than the launches
+// Is an FP64 cycle on a level in list order, which works on the caller's
+// vectors, worth the copies to own_c and own_b and back that a replay takes?
+// Jacobi cycles of 2D grids, several contexts at once, launched / replayed:
+// levels in k_coarse_down and k_coarse_up up to the top (33^2) 25 / 50 us; one
+// level above them (65^2) V(1,1) 47 / 52 us, V(2,2) 55 / 53, V(3,3) 63 / 54;
+// two (97^2) V(1,1) 65 / 56.  From 256^2 on the device takes longer than the
+// host.
 constexpr size_t kOwnCycleValues = 65536;
+int launched_above(const ugmg_ctx *ctx) {
+  return ctx->p.gamma == 1 ? std::max(ctx->bl, ctx->fuse_top[0]) : ctx->bl;
+}
+bool replay_pays(const ugmg_ctx *ctx, int level) {
+  const DevLevel &d = ctx->dev[level];
+  return (size_t)d.n * d.nb <= ctx->own_n &&
+         (level - launched_above(ctx)) * (ctx->p.nu1 + ctx->p.nu2 + 3) >= 7;
+}
 
 // ------------------------------------------------------------ BCGSSolver
 // Work of BCGSSolver (np/procs/ls.cc:1864-2062) on nb columns of level
@@ -1894,6 +1925,16 @@ int prep_device(ugmg_ctx *ctx, PrepState &ps) {
       fill(c64[l], double());
       fill(c32[l], float());
     }
+    size_t own = 0;
+    for (int l = launched_above(ctx) + 1; l <= level; ++l) {
+      const size_t nv = (size_t)ctx->dev[l].n * ctx->dev[l].nb;
+      if (!ctx->dev[l].perm && !ctx->grouped && nv <= kOwnCycleValues) own = std::max(own, nv);
+    }
+    if (own) {
+      if ((rc = dalloc(ctx, &ctx->own_c, 2 * own))) return rc;
+      ctx->own_b = ctx->own_c + own;
+      ctx->own_n = own;
+    }
     if ((rc = upload(ctx, &ctx->clev64, c64.data(), c64.size()))) return rc;
     if ((rc = upload(ctx, &ctx->clev32, c32.data(), c32.size()))) return rc;
     ctx->part_cap = std::max(1024, (max_slices + 3) / 4 + 1);
@@ -2614,9 +2655,13 @@ int ugmg_iter(ugmg_ctx *ctx, int level, double *c, double *b) {
   if (rc) return rc;
   if (base_singular(ctx)) return fail(ctx, UGMG_E_SINGULAR, "zero pivot in the band LU of the base level");
   DevLevel &d = ctx->dev[level];
-  if (ctx->p.precision == UGMG_MIXED) {
+  const bool mixed = ctx->p.precision == UGMG_MIXED, list = !d.perm && !mixed;
+  double *oc = mixed ? nullptr : list ? ctx->own_c : d.c, *ob = mixed ? nullptr : list ? ctx->own_b : d.b;
+  bool replay = false;
+  if ((!list || replay_pays(ctx, level)) && (rc = replayed(ctx, level, oc, replay))) return rc;
+  if (mixed) {
     to_dev<float, double>(ctx, level, b, d.vs, d.b32);
-    if ((rc = own_cycle(ctx, level))) return rc;
+    if ((rc = own_cycle(ctx, level, oc, ob, replay))) return rc;
     if (!d.perm) {
       launch_convert<double, float>(ctx->stream, d.n * d.nb, d.c32, c, 1, d.vs, d.vs);
       launch_spmv<double, double, double>(ctx->stream, d.A.d64(), 0, d.A.nslices, c, b, nullptr, 0, d.nt, B1(d));
@@ -2627,13 +2672,13 @@ int ugmg_iter(ugmg_ctx *ctx, int level, double *c, double *b) {
       to_user<double, double>(ctx, level, d.c, c, d.vs);
       to_user<double, double>(ctx, level, d.b, b, d.vs);
     }
-  } else if (!d.perm && (!can_capture(ctx) || (size_t)d.n * d.nb > kOwnCycleValues)) {
+  } else if (list && !replay) {
     lmgc<double>(ctx, level, c, b, 0);
   } else {
-    to_dev<double, double>(ctx, level, b, d.vs, d.b);
-    if ((rc = own_cycle(ctx, level))) return rc;
-    to_user<double, double>(ctx, level, d.c, c, d.vs);
-    to_user<double, double>(ctx, level, d.b, b, d.vs);
+    to_dev<double, double>(ctx, level, b, d.vs, ob);
+    if ((rc = own_cycle(ctx, level, oc, ob, replay))) return rc;
+    to_user<double, double>(ctx, level, oc, c, d.vs);
+    to_user<double, double>(ctx, level, ob, b, d.vs);
   }
   HIPCHK(hipGetLastError());
   return UGMG_OK;
@@ -3173,15 +3218,20 @@ int ugmg_iter_batch(ugmg_ctx *ctx, int level, int nrhs, double *c, double *b, in
   hipStream_t st = ctx->stream;
   ctx->nb = nrhs;
   const Batch bt = batch(ctx, level);
+  bool replay = false;
+  if ((rc = replayed(ctx, level, ctx->p.precision == UGMG_MIXED ? nullptr : d.c, replay))) {
+    ctx->nb = 1;
+    return rc;
+  }
   if (ctx->p.precision == UGMG_MIXED) {
     to_dev<float, double>(ctx, level, b, ld, d.b32, nrhs);
-    rc = own_cycle(ctx, level);
+    rc = own_cycle(ctx, level, nullptr, nullptr, replay);
     launch_convert<double, float>(st, d.n * d.nb, d.c32, d.c, nrhs, d.vs, d.vs);
     to_dev<double, double>(ctx, level, b, ld, d.b, nrhs);
     launch_spmv<double, double, double>(st, d.A.d64(), 0, d.A.nslices, d.c, d.b, nullptr, 0, d.nt, bt);
   } else {
     to_dev<double, double>(ctx, level, b, ld, d.b, nrhs);
-    rc = own_cycle(ctx, level);
+    rc = own_cycle(ctx, level, d.c, d.b, replay);
   }
   to_user<double, double>(ctx, level, d.c, c, ld, nrhs);
   to_user<double, double>(ctx, level, d.b, b, ld, nrhs);
