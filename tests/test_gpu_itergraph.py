@@ -58,6 +58,52 @@ def test_iter_calls(kw):
         ctx.close()
 
 
+@pytest.mark.parametrize("kw", [dict(smoother=ugmg.SMOOTH_JAC, damp=0.8), dict(), dict(precision=ugmg.MIXED)])
+def test_calls_that_do_not_wait(kw):
+    """Alternating levels and columns, more of them than graphs are kept for,
+    solves and new parameters in between, with nothing waiting for the GPU:
+    no graph goes while it runs."""
+    P = problems.q1(2, 3, 4, problems.KAPPA_JUMP, seed=2)
+    calls = [(4, 1), (4, 3), (4, 1), (4, 3), (4, 0), (4, 1), (3, 2), (4, 3), (3, 2), (3, 1), (4, 1), (3, 1), (2, 3),
+             (2, 2), (2, 1), (2, 3), (2, 2), (2, 1), (4, 2), (3, 3), (4, 2), (3, 3), (4, 1), (4, 0)]
+    out = []
+    for use in (0, 1):
+        ctx = ugmg.Context(0)
+        ctx.set_stream(torch.cuda.Stream())
+        ctx.set_hierarchy(P)
+        ctx.set_batch(3)
+
+        def params(nu):
+            ctx.set_params(**{**dict(nu1=nu, nu2=nu, gamma=1, baselevel=1, smoother=ugmg.SMOOTH_GS, damp=1.0,
+                                     base_abslimit=1e-300, base_maxiter=1, use_graph=use), **kw})
+
+        params(2)
+        ctx.preprocess()
+        bufs = []
+        for k in range(3 * len(calls)):
+            level, cols = calls[k % len(calls)]
+            f = torch.from_numpy(np.random.default_rng(k).uniform(-1.0, 1.0, (max(cols, 1), P.levels[level].n))).cuda()
+            bufs.append((level, cols, torch.zeros_like(f), f))
+        xs = torch.zeros(P.levels[-1].n, dtype=torch.float64, device="cuda")
+        rhs = torch.from_numpy(P.rhs).cuda()
+        torch.cuda.synchronize()
+        for k, (level, cols, c, b) in enumerate(bufs):
+            if cols != 1:
+                ctx.iter_batch(level, c, b)
+            else:
+                ctx.iter(level, c[0], b[0])
+            if k % 17 == 16:
+                params(1 + k % 3)
+            if k == len(calls):
+                ctx.solve(P.top, xs, rhs, red=1e-4, maxiter=5)
+        ctx.sync()
+        out.append([v.cpu().numpy() for _, _, c, b in bufs for v in (c, b)])
+        ctx.close()
+    assert all(np.any(v) and np.all(np.isfinite(v)) for v in out[0])
+    for k, (a, b) in enumerate(zip(*out)):
+        assert np.array_equal(a, b), k
+
+
 @pytest.mark.parametrize("kw", [
     dict(smoother=ugmg.SMOOTH_JAC, damp=0.8), dict(smoother=ugmg.SMOOTH_JAC, damp=0.8, nu1=2, nu2=2), dict(),
     dict(precision=ugmg.MIXED)])

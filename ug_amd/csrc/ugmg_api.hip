@@ -233,14 +233,18 @@ struct ugmg_ctx {
   static constexpr int kMaxGraphs = 65;
   hipGraphExec_t gexec[kMaxGraphs] = {};
   int gkind = -1, glevel = -1;
-  // the cycle of ugmg_iter and ugmg_iter_batch on a level and vectors of the
-  // context (c; null: FP32): its graph, and the calls it has served (the
-  // first one records nothing)
+  // the cycles of ugmg_iter and ugmg_iter_batch, by level, columns and vectors
+  // of the context (c; null: FP32): each one's graph, recorded by its second
+  // call.  The first kIterGraphs stay, later ones are launched.
   struct IterGraph {
     hipGraphExec_t g = nullptr;
-    int level = -1, nb = 0, calls = 0;
+    int level = -1, nb = 0;
     const double *c = nullptr;
-  } ig;
+  };
+  static constexpr int kIterGraphs = 8;
+  std::vector<IterGraph> ig;
+  // graphs dropped while the stream was being captured
+  std::vector<hipGraphExec_t> ig_dropped;
   // ugmg_iter's on levels in list order, where launches work on the caller's
   // vectors: not the level's own, whose b a restriction adds to
   double *own_c = nullptr, *own_b = nullptr;
@@ -466,7 +470,27 @@ void free_device(ugmg_ctx *ctx) {
   ctx->top = -1;
 }
 
-void drop_graph(ugmg_ctx *ctx) {
+// ugmg_iter returns without waiting, so the stream is waited for before its
+// graphs go (the solves wait after every replay).  A stream that is being
+// captured cannot be: then they stay until ugmg_destroy.
+void drop_iter_graphs(ugmg_ctx *ctx) {
+  bool replayed = false;
+  for (auto &e : ctx->ig) replayed |= e.g != nullptr;
+  if (replayed) {
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    hipError_t e = hipStreamIsCapturing(ctx->stream, &cs);
+    if (e == hipSuccess && cs == hipStreamCaptureStatusNone) e = hipStreamSynchronize(ctx->stream);
+    const bool waited = e == hipSuccess && cs == hipStreamCaptureStatusNone;
+    if (e != hipSuccess) (void)hipGetLastError();   // (a stream that is gone)
+    for (auto &i : ctx->ig)
+      if (i.g && waited) hipGraphExecDestroy(i.g);
+      else if (i.g) ctx->ig_dropped.push_back(i.g);
+  }
+  ctx->ig.clear();
+}
+
+// the graphs on a solve's vectors
+void drop_solve_graphs(ugmg_ctx *ctx) {
   for (hipGraphExec_t &g : ctx->gexec)
     if (g) {
       hipGraphExecDestroy(g);
@@ -479,9 +503,12 @@ void drop_graph(ugmg_ctx *ctx) {
       g = nullptr;
     }
   ctx->sgkind = -1;
-  if (ctx->ig.g) hipGraphExecDestroy(ctx->ig.g);
-  ctx->ig = ugmg_ctx::IterGraph();
   drop_bcgs_graphs(ctx);
+}
+
+void drop_graph(ugmg_ctx *ctx) {
+  drop_solve_graphs(ctx);
+  drop_iter_graphs(ctx);
 }
 
 inline int packed_ident(const ugmg_ctx *ctx) {
@@ -909,7 +936,7 @@ int launch_iteration(ugmg_ctx *ctx, int level, double *x, double *b, int cycles)
   } else {
     const int kind = ctx->p.precision;
     if (ctx->gkind != kind || ctx->glevel != level || ctx->gx != x || ctx->gb != b) {
-      drop_graph(ctx);
+      drop_solve_graphs(ctx);
       ctx->gkind = kind;
       ctx->glevel = level;
       ctx->gx = x;
@@ -1112,31 +1139,37 @@ double iteration_bytes(const ugmg_ctx *ctx, int l, int cycles) {
   return by + d.A.bytes(8) + (double)d.n * d.nb * (4.0 + 4.0 + 16.0 + 16.0 + 4.0) + d.n;
 }
 
-// Is this call's cycle to be replayed from a graph?  From the second call
-// with the same level, columns and c (own_cycle's) on: a launch per operation takes the
-// host 2.3 to 3 us, as long as small levels take the device or longer (8
-// columns of 33^3: 307 us a call, 187 us replayed).  A stream that is being
-// captured gets the launches.
-int replayed(ugmg_ctx *ctx, int level, const double *c, bool &yes) {
-  yes = false;
+// The graph that this call's cycle is to be replayed from, or null.  It is
+// recorded by the second call with the same level, columns and c
+// (own_cycle's): a launch per operation takes the host 2.3 to 3 us, as long
+// as small levels take the device or longer (8 columns of 33^3: 307 us a
+// call, 187 us replayed).  Recording takes about 10 us an operation, once
+// (17^2: 0.1 ms, 65^3: 0.4 to 1.1 ms).  A stream that is being captured gets the
+// launches.
+int iter_graph(ugmg_ctx *ctx, int level, const double *c, ugmg_ctx::IterGraph *&out) {
+  out = nullptr;
   if (!can_capture(ctx)) return 0;
-  auto &ig = ctx->ig;
   hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
   HIPCHK(hipStreamIsCapturing(ctx->stream, &cs));
-  if (ig.level != level || ig.nb != ctx->nb || ig.c != c) {
-    if (ig.g) hipGraphExecDestroy(ig.g);
-    ig = ugmg_ctx::IterGraph();
-    ig.level = level;
-    ig.nb = ctx->nb;
-    ig.c = c;
+  if (cs != hipStreamCaptureStatusNone) return 0;
+  for (auto &e : ctx->ig)
+    if (e.level == level && e.nb == ctx->nb && e.c == c) {
+      out = &e;
+      return 0;
+    }
+  if ((int)ctx->ig.size() < ugmg_ctx::kIterGraphs) {
+    try {
+      ctx->ig.push_back({nullptr, level, ctx->nb, c});
+    } catch (const std::bad_alloc &) {
+      return fail(ctx, UGMG_E_NOMEM, "host allocation");
+    }
   }
-  yes = cs == hipStreamCaptureStatusNone && ig.calls++ > 0;
   return 0;
 }
 
 // The cycle of ugmg_iter on c and b, vectors of the context, or (mixed, both
-// null) inner_cycles of them on the level's FP32 vectors
-int own_cycle(ugmg_ctx *ctx, int level, double *c, double *b, bool replay) {
+// null) inner_cycles of them on the level's FP32 vectors; from `ig` if given
+int own_cycle(ugmg_ctx *ctx, int level, double *c, double *b, ugmg_ctx::IterGraph *ig) {
   DevLevel &d = ctx->dev[level];
   auto enqueue = [&] {
     if (ctx->p.precision == UGMG_MIXED) {
@@ -1146,25 +1179,24 @@ int own_cycle(ugmg_ctx *ctx, int level, double *c, double *b, bool replay) {
       lmgc<double>(ctx, level, c, b, 0);
     }
   };
-  auto &ig = ctx->ig;
-  if (!replay) {
+  if (!ig) {
     enqueue();
     HIPCHK(hipGetLastError());
     return 0;
   }
-  if (!ig.g) {
+  if (!ig->g) {
     hipGraph_t g = nullptr;
     HIPCHK(hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeThreadLocal));
     enqueue();
     HIPCHK(hipStreamEndCapture(ctx->stream, &g));
-    hipError_t e = hipGraphInstantiate(&ig.g, g, nullptr, nullptr, 0);
+    hipError_t e = hipGraphInstantiate(&ig->g, g, nullptr, nullptr, 0);
     hipGraphDestroy(g);
     if (e != hipSuccess) {
-      ig.g = nullptr;
+      ig->g = nullptr;
       return fail(ctx, UGMG_E_HIP, std::string("hipGraphInstantiate: ") + hipGetErrorString(e));
     }
   }
-  HIPCHK(hipGraphLaunch(ig.g, ctx->stream));
+  HIPCHK(hipGraphLaunch(ig->g, ctx->stream));
   return 0;
 }
 
@@ -2015,6 +2047,8 @@ int ugmg_destroy(ugmg_ctx *ctx) {
   hipSetDevice(ctx->device);
   if (ctx->stream) hipStreamSynchronize(ctx->stream);
   free_device(ctx);
+  if (!ctx->ig_dropped.empty()) hipDeviceSynchronize();
+  for (hipGraphExec_t g : ctx->ig_dropped) hipGraphExecDestroy(g);
   for (int l = 0; l < (int)ctx->dcsr.size(); ++l) drop_dcsr(ctx, l);
   if (ctx->red_host) hipHostFree(ctx->red_host);
   if (ctx->surf_sq_host) hipHostFree(ctx->surf_sq_host);
@@ -2657,11 +2691,11 @@ int ugmg_iter(ugmg_ctx *ctx, int level, double *c, double *b) {
   DevLevel &d = ctx->dev[level];
   const bool mixed = ctx->p.precision == UGMG_MIXED, list = !d.perm && !mixed;
   double *oc = mixed ? nullptr : list ? ctx->own_c : d.c, *ob = mixed ? nullptr : list ? ctx->own_b : d.b;
-  bool replay = false;
-  if ((!list || replay_pays(ctx, level)) && (rc = replayed(ctx, level, oc, replay))) return rc;
+  ugmg_ctx::IterGraph *ig = nullptr;
+  if ((!list || replay_pays(ctx, level)) && (rc = iter_graph(ctx, level, oc, ig))) return rc;
   if (mixed) {
     to_dev<float, double>(ctx, level, b, d.vs, d.b32);
-    if ((rc = own_cycle(ctx, level, oc, ob, replay))) return rc;
+    if ((rc = own_cycle(ctx, level, oc, ob, ig))) return rc;
     if (!d.perm) {
       launch_convert<double, float>(ctx->stream, d.n * d.nb, d.c32, c, 1, d.vs, d.vs);
       launch_spmv<double, double, double>(ctx->stream, d.A.d64(), 0, d.A.nslices, c, b, nullptr, 0, d.nt, B1(d));
@@ -2672,11 +2706,11 @@ int ugmg_iter(ugmg_ctx *ctx, int level, double *c, double *b) {
       to_user<double, double>(ctx, level, d.c, c, d.vs);
       to_user<double, double>(ctx, level, d.b, b, d.vs);
     }
-  } else if (list && !replay) {
+  } else if (list && !ig) {
     lmgc<double>(ctx, level, c, b, 0);
   } else {
     to_dev<double, double>(ctx, level, b, d.vs, ob);
-    if ((rc = own_cycle(ctx, level, oc, ob, replay))) return rc;
+    if ((rc = own_cycle(ctx, level, oc, ob, ig))) return rc;
     to_user<double, double>(ctx, level, oc, c, d.vs);
     to_user<double, double>(ctx, level, ob, b, d.vs);
   }
@@ -3190,7 +3224,7 @@ int ugmg_solve_host(ugmg_ctx *ctx, int level, double *x, double *b, const double
   if (!rc && (hipMemcpy(x, dx, bytes, hipMemcpyDeviceToHost) != hipSuccess ||
               hipMemcpy(b, db, bytes, hipMemcpyDeviceToHost) != hipSuccess))
     rc = fail(ctx, UGMG_E_HIP, "copy out");
-  drop_graph(ctx);
+  drop_solve_graphs(ctx);
   hipFree(dx);
   hipFree(db);
   return rc;
@@ -3218,20 +3252,20 @@ int ugmg_iter_batch(ugmg_ctx *ctx, int level, int nrhs, double *c, double *b, in
   hipStream_t st = ctx->stream;
   ctx->nb = nrhs;
   const Batch bt = batch(ctx, level);
-  bool replay = false;
-  if ((rc = replayed(ctx, level, ctx->p.precision == UGMG_MIXED ? nullptr : d.c, replay))) {
+  ugmg_ctx::IterGraph *ig = nullptr;
+  if ((rc = iter_graph(ctx, level, ctx->p.precision == UGMG_MIXED ? nullptr : d.c, ig))) {
     ctx->nb = 1;
     return rc;
   }
   if (ctx->p.precision == UGMG_MIXED) {
     to_dev<float, double>(ctx, level, b, ld, d.b32, nrhs);
-    rc = own_cycle(ctx, level, nullptr, nullptr, replay);
+    rc = own_cycle(ctx, level, nullptr, nullptr, ig);
     launch_convert<double, float>(st, d.n * d.nb, d.c32, d.c, nrhs, d.vs, d.vs);
     to_dev<double, double>(ctx, level, b, ld, d.b, nrhs);
     launch_spmv<double, double, double>(st, d.A.d64(), 0, d.A.nslices, d.c, d.b, nullptr, 0, d.nt, bt);
   } else {
     to_dev<double, double>(ctx, level, b, ld, d.b, nrhs);
-    rc = own_cycle(ctx, level, d.c, d.b, replay);
+    rc = own_cycle(ctx, level, d.c, d.b, ig);
   }
   to_user<double, double>(ctx, level, d.c, c, ld, nrhs);
   to_user<double, double>(ctx, level, d.b, b, ld, nrhs);
@@ -3885,7 +3919,7 @@ int launch_group_iteration(ugmg_ctx *ctx, int top, double *x, double *b, int w, 
     HIPCHK(hipGetLastError());
   } else {
     if (ctx->gkind != -2 || ctx->glevel != top || ctx->gx != x || ctx->gb != b) {
-      drop_graph(ctx);
+      drop_solve_graphs(ctx);
       ctx->gkind = -2;
       ctx->glevel = top;
       ctx->gx = x;
