@@ -385,12 +385,13 @@ def test_base_levels_and_base_iterations(jump3d_33, bl, maxit):
 
 
 def test_fused_coarse_cycle_matches(poisson2d, monkeypatch):
-    """The single-workgroup coarse-cycle kernel (levels up to UGMG_FUSE_ROWS
-    vectors) gives the oracle's defects, W-cycle (gamma 2) included."""
+    """Levels of up to UGMG_FUSE_ROWS vectors in one workgroup per column give
+    the oracle's defects with both smoothers; a W-cycle (gamma 2), which gets a
+    launch per operation whatever UGMG_FUSE_ROWS says, too."""
     from ug_amd import ugmg
     H = O.Hierarchy(poisson2d.levels)
     monkeypatch.setenv("UGMG_FUSE_ROWS", "5000")
-    for gamma, sm in ((1, ugmg.SMOOTH_JAC), (2, ugmg.SMOOTH_GS)):
+    for gamma, sm in ((1, ugmg.SMOOTH_JAC), (1, ugmg.SMOOTH_GS), (2, ugmg.SMOOTH_GS)):
         osm = O.JAC if sm == ugmg.SMOOTH_JAC else O.MCGS
         damp = 0.8 if sm == ugmg.SMOOTH_JAC else 1.0
         want = O.ls_solve(H, poisson2d.top, O.params(smoother=osm, damp=damp, baselevel=0, gamma=gamma),

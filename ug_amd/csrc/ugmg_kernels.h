@@ -11,7 +11,6 @@
 
 namespace ugmg {
 
-constexpr int kMaxLevels = 32;
 constexpr int kMaxColors = 32;
 constexpr int kCoarseThreads = 1024;
 
