@@ -1,7 +1,8 @@
-"""Batches of at least four columns on rows of at most 8 entries take several
-columns per thread: cycles and BiCGStab give every column the bits it gets
-alone, with full and partial groups of columns, GS and Jacobi levels, uniform
-and explicit slices, both precisions."""
+"""Large batches of at least four columns on rows of at most 8 entries take
+several columns per thread (here, with UGMG_MC_WAVES=0, small ones too, but for
+5 columns, whose second group would be mostly empty): cycles and BiCGStab give
+every column the bits it gets alone, with full and partial groups of columns,
+GS and Jacobi levels, uniform and explicit slices, both precisions."""
 import numpy as np
 import pytest
 
@@ -25,12 +26,13 @@ def _context(P, cols, **kw):
     return ctx, torch.from_numpy(f).cuda()
 
 
-@pytest.mark.parametrize("cols", [4, 5, 7, 8])
+@pytest.mark.parametrize("cols", [4, 5, 6, 7, 8, 13])
 @pytest.mark.parametrize("which,kw", [
     ("cd", {}), ("cd", dict(precision=ugmg.MIXED, damp=0.9)), ("local", dict(baselevel=1)),
     ("q1", dict(smoother=ugmg.SMOOTH_JAC, damp=0.8))])
 def test_columns_of_a_cycle(which, kw, cols, monkeypatch):
     monkeypatch.setenv("UGMG_FUSE_ROWS", "0")     # the launches, on small levels too
+    monkeypatch.setenv("UGMG_MC_WAVES", "0")
     P = {"cd": lambda: problems.p1_cd(5, 1e-3, float("nan"), seed=1), "local": lambda: problems.p1_local(4, 2),
          "q1": lambda: problems.q1(3, 1, 4, problems.KAPPA_JUMP, seed=2)}[which]()
     print(f"columns {which} {cols}", flush=True)
@@ -51,9 +53,10 @@ def test_columns_of_a_cycle(which, kw, cols, monkeypatch):
     ctx.close()
 
 
-@pytest.mark.parametrize("cols", [4, 6])
+@pytest.mark.parametrize("cols", [4, 6, 13])
 @pytest.mark.parametrize("precision", [ugmg.FP64, ugmg.MIXED])
-def test_columns_of_bicgstab(precision, cols):
+def test_columns_of_bicgstab(precision, cols, monkeypatch):
+    monkeypatch.setenv("UGMG_MC_WAVES", "0")
     P = problems.p1_cd(5, 1e-3, float("nan"), seed=3)
     print(f"bicgstab columns {cols}", flush=True)
     ctx, f = _context(P, cols, precision=precision, nu2=1)

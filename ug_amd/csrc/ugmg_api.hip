@@ -297,6 +297,9 @@ struct ugmg_ctx {
   // folded sweeps with the upper and lower row products on two wavefronts
   // per slice (UGMG_GS_SPLIT=0: one wavefront per slice)
   bool gs_split = true;
+  // wavefronts from which a batched launch takes four columns per thread
+  // (UGMG_MC_WAVES)
+  int mc_waves = kMcWaves;
   // BCGSSolver work (allocated on first use, freed with the hierarchy)
   struct Bcgs {
     int nrhs = 0, maxdef = 0, npart = 0;
@@ -521,6 +524,7 @@ inline Batch batch(const ugmg_ctx *ctx, int l) {
   const DevLevel &d = ctx->dev[l];
   Batch bt{ctx->nb, d.vs, d.nb, d.dms, ctx->base_ims, d.vt, d.ntypes};
   bt.idents = packed_ident(ctx);
+  bt.mc_waves = ctx->mc_waves;
   return bt;
 }
 inline Batch B1(const DevLevel &d) { return Batch{1, d.vs, d.nb, 0, 0, d.vt, d.ntypes}; }
@@ -868,7 +872,7 @@ void lmgc(ugmg_ctx *ctx, int l, T *c, T *b, int cmode, bool c0_done = false) {
     launch_scale_comp<T>(st, d.n, d.nb, p.lmgc_damp, t, c, 1, batch(ctx, l));
   } else {
     launch_interp<T>(st, d.P.d<T>(), d.iskip, dc.cv<T>(), (T)p.lmgc_damp[0], t, c, d.ntv<T>(), nb, d.vs,
-                     dc.vs, d.nb);
+                     dc.vs, d.nb, ctx->mc_waves);
   }
   if (fold_colour0(ctx, l, p.nu2, true)) {
     post_smooth_folded<T>(ctx, l, t, b, c, p.nu2);
@@ -1484,6 +1488,8 @@ int prep_host(ugmg_ctx *ctx, int level, PrepState &ps) {
   ctx->fuse_steps = !(env_gsf && std::atoi(env_gsf) == 0);
   const char *env_split = std::getenv("UGMG_GS_SPLIT");
   ctx->gs_split = !(env_split && std::atoi(env_split) == 0);
+  const char *env_mc = std::getenv("UGMG_MC_WAVES");
+  ctx->mc_waves = env_mc ? std::atoi(env_mc) : kMcWaves;
   const char *env_fuse = std::getenv("UGMG_FUSE_ROWS");
   ps.fuse_rows = env_fuse ? std::atoi(env_fuse) : kCoarseRows;
   ps.level = level;

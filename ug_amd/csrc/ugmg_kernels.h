@@ -70,6 +70,10 @@ struct CoarseArgs {
 // LDS of a workgroup: three vectors of a level and one of the level below
 constexpr size_t kCoarseLds = 160 * 1024;
 
+// a batched launch takes four columns per thread where that leaves at least
+// this many wavefronts: three per SIMD (mc_columns)
+constexpr int kMcWaves = 3072;
+
 // Batched launches: every vector argument holds `nrhs` columns, column j at
 // offset j * vs (vs = the level's column stride, >= n); the column index of a
 // workgroup is its second grid coordinate.  nrhs = 1 is the plain case.
@@ -97,6 +101,7 @@ struct Batch {
     double d[4] = {};
     int vb = 0;
   } pdamp;
+  int mc_waves = kMcWaves;
 };
 
 // t[v b + q] *= d[q] on n vectors of b components, then (c non-null) c =
@@ -233,7 +238,7 @@ int launch_dot_part(hipStream_t st, int n, const T *x, const uint8_t *vclass, do
                     Batch bt);
 template <typename T>
 void launch_interp(hipStream_t st, const DSell<T> &P, const uint32_t *fskip, const T *cc, T damp,
-                   T *t, T *c, bool nt, int nrhs, size_t vsf, size_t vsc, int b);
+                   T *t, T *c, bool nt, int nrhs, size_t vsf, size_t vsc, int b, int mc_waves = kMcWaves);
 int reduce_parts(int n);
 template <typename T>
 void launch_dot(hipStream_t st, int n, const T *x, const T *y, const uint8_t *vclass,

@@ -761,12 +761,10 @@ __global__ __launch_bounds__(kBlock) void k_interp(DSell<T> P, int nsl,
 
 // ------------------------------------------------- several columns a row
 // The kernels above with kMc columns of a batch per thread, for one matrix
-// and rows of at most 8 entries (one round of loads).  A workgroup per column
-// reads the entries again from L2 for each and has one column's gathers in
-// flight: 2 TB/s on 32 columns of 513^2.  Sums in the same order, column by
-// column.  BiCGStab on 32 columns of 513^2 21.1 -> 17.7 ms.  Wider rows stay
-// with a workgroup per column: kMc columns of 27 gathers do not fit the
-// registers in one round, and their few workgroups wait for latency.
+// and rows of at most 8 entries (one round of loads), where enough wavefronts
+// are left (mc_columns).  A workgroup per column reads the entries again from
+// L2 for each and has one column's gathers in flight.  Sums in the same order,
+// column by column.  BiCGStab on 32 columns of 513^2 26.9 -> 21.4 ms (mixed).
 constexpr int kMc = 4;
 // the thread's columns col_ .. col_ + nc - 1
 #define MC_COLUMNS(nrhs)                  \
@@ -1769,12 +1767,23 @@ static dim3 slab_grid(const DSell<TV> &S, int slice0, int nsl, int nrhs) {
     }                        \
   } while (0)
 
-// may a batched launch over S take kMc columns a thread?
-template <typename TV>
-static bool mc_columns(const DSell<TV> &S, int wmax, int nrhs) {
-  return nrhs >= kMc && wmax <= 8 && S.mst == 0 && S.dms == 0;
-}
 static int mc_groups(int nrhs) { return (nrhs + kMc - 1) / kMc; }
+// Does a batched launch over nsl slices of S take kMc columns a thread?  A
+// quarter of the wavefronts is left: three a SIMD are enough to hide the
+// loads, fewer are not.  One column a thread / kMc: colour sweeps of 1028
+// slices (2D Q1 V(1,1) cycles on 513^2) with 4 columns 195 / 209 us, 9 331 /
+// 334, 13 451 / 432; 257 slices with 16 columns 155 / 163, 32 352 / 354; 4112
+// slices with 4 597 / 540.  A last group that is mostly empty costs more than
+// the others gain (5 columns of 513^2 308 / 358), so at most a third more
+// columns than there are.  9 entries (2D Q1 rows, two rounds of loads; levels
+// past 64 MB aside, which gain 5 %) gain nothing (8 columns of 513^2 295 /
+// 296); kMc columns of 27 gathers do not fit the registers.
+template <typename TV>
+static bool mc_columns(const DSell<TV> &S, int nsl, int wmax, int nrhs, int mc_waves) {
+  const int groups = mc_groups(nrhs);
+  return nrhs >= kMc && 3 * kMc * groups <= 4 * nrhs && (long long)nsl * groups >= mc_waves && wmax <= 8 &&
+         S.mst == 0 && S.dms == 0;
+}
 
 template <typename TV, typename TX, typename TY>
 void launch_spmv(hipStream_t st, const DSell<TV> &A, int slice0, int nsl, const TX *x, TY *y,
@@ -1833,7 +1842,7 @@ template <typename TV, typename T>
 void launch_spmv_c0(hipStream_t st, const DSell<TV> &A, const T *x, T *y, const T *diag, T *u,
                     int ncs0, bool nt, Batch bt) {
   if (A.nslices <= 0) return;
-  if (mc_columns(A, A.wmax, bt.nrhs)) {
+  if (mc_columns(A, A.nslices, A.wmax, bt.nrhs, bt.mc_waves)) {
     NT_DISPATCH(nt, k_spmv_c0_mc<T, NTV><<<slab_grid(A, 0, A.nslices, mc_groups(bt.nrhs)), kBlock, 0, st>>>(
                         A, A.nslices, bt.nrhs, x, y, diag, u, ncs0, bt.vs));
     return;
@@ -1911,7 +1920,7 @@ void launch_gs_color(hipStream_t st, const DSell<TV> &L, int slice0, int nsl, in
                                                             L, slice0, nsl, b, diag, vclass, v, bt.vs))));
     return;
   }
-  if (mc_columns(L, wmax, bt.nrhs)) {
+  if (mc_columns(L, nsl, wmax, bt.nrhs, bt.mc_waves)) {
     const int nrhs = bt.nrhs;
     bt.nrhs = mc_groups(nrhs);     // (the grid of GSB_DISPATCH)
     GSB_DISPATCH(nsl, NT_DISPATCH(nt, k_gs_color_mc<T, NTV, BSV><<<g, BSV, 0, st>>>(L, slice0, nsl, nrhs, b, diag, vclass,
@@ -2031,7 +2040,7 @@ void launch_gs_defect(hipStream_t st, const DSell<TV> &U, const T *v, T *b, cons
                         U, U.nslices, v, b, vclass, damp, c, xout, bt.vs)));
     return;
   }
-  if (mc_columns(U, U.wmax, bt.nrhs) && c && !xout) {
+  if (mc_columns(U, U.nslices, U.wmax, bt.nrhs, bt.mc_waves) && c && !xout) {
     const dim3 gm = slab_grid(U, 0, U.nslices, mc_groups(bt.nrhs));
     NT_DISPATCH(nt, if (cmode == 0) k_gs_defect_mc<T, 0, NTV><<<gm, kBlock, 0, st>>>(
                         U, U.nslices, bt.nrhs, v, b, vclass, damp, c, bt.vs);
@@ -2326,7 +2335,7 @@ int launch_dot_part(hipStream_t st, int n, const T *x, const uint8_t *vclass, do
 
 template <typename T>
 void launch_interp(hipStream_t st, const DSell<T> &P, const uint32_t *fskip, const T *cc, T damp,
-                   T *t, T *c, bool nt, int nrhs, size_t vsf, size_t vsc, int b) {
+                   T *t, T *c, bool nt, int nrhs, size_t vsf, size_t vsc, int b, int mc_waves) {
   if (P.nslices <= 0) return;
   const dim3 g = grid2(nblk_slices(P.nslices), nrhs);
   if (b > 1 && P.bb > 1) {
@@ -2343,7 +2352,7 @@ void launch_interp(hipStream_t st, const DSell<T> &P, const uint32_t *fskip, con
                                                                                     damp, t, c, vsf, vsc)));
     return;
   }
-  if (mc_columns(P, P.wmax, nrhs)) {
+  if (mc_columns(P, P.nslices, P.wmax, nrhs, mc_waves)) {
     const dim3 gm = grid2(nblk_slices(P.nslices), mc_groups(nrhs));
     NT_DISPATCH(nt, if (c) k_interp_mc<T, 1, NTV><<<gm, kBlock, 0, st>>>(P, P.nslices, nrhs, fskip, cc, damp, t, c, vsf, vsc);
                 else k_interp_mc<T, 0, NTV><<<gm, kBlock, 0, st>>>(P, P.nslices, nrhs, fskip, cc, damp, t, c, vsf, vsc));
@@ -2363,10 +2372,10 @@ void launch_interp(hipStream_t st, const DSell<T> &P, const uint32_t *fskip, con
 }
 template void launch_interp<double>(hipStream_t, const DSell<double> &, const uint32_t *,
                                     const double *, double, double *, double *, bool, int,
-                                    size_t, size_t, int);
+                                    size_t, size_t, int, int);
 template void launch_interp<float>(hipStream_t, const DSell<float> &, const uint32_t *,
                                    const float *, float, float *, float *, bool, int, size_t,
-                                   size_t, int);
+                                   size_t, int, int);
 
 int reduce_parts(int n) {
   int g = nblk(n);
@@ -2838,7 +2847,7 @@ void launch_bcgs_spmv(hipStream_t st, const DSell<double> &A, const TQ *q, doubl
   const dim3 g = grid2(nblk_slices(A.nslices), bt.nrhs);
   DSell<double> Ap = A;
   Ap.ncb = 0;   // its partial sums are strided by the grid: the plain map
-  if (mc_columns(A, A.wmax, bt.nrhs)) {
+  if (mc_columns(A, A.nslices, A.wmax, bt.nrhs, bt.mc_waves)) {
     NT_DISPATCH(nt, k_bcgs_spmv_mc<TQ, NTV><<<grid2(nblk_slices(A.nslices), mc_groups(bt.nrhs)), kBlock, 0, st>>>(
                         Ap, A.nslices, bt.nrhs, q, y, z, vclass, part, yy, skip_half, s, bt.vs));
     return;
