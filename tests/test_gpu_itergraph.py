@@ -1,6 +1,7 @@
 """ugmg_iter and ugmg_iter_batch replay their cycle from a graph from the
-second call on (use_graph): every call, with other vectors and changing
-levels, columns and parameters in between, gives the bits of launches."""
+second call on (use_graph), where it is enough launches: every call, with other
+vectors and changing levels, columns and parameters in between, gives the bits
+of launches."""
 import numpy as np
 import pytest
 
@@ -59,10 +60,11 @@ def test_iter_calls(kw):
 
 
 @pytest.mark.parametrize("kw", [dict(smoother=ugmg.SMOOTH_JAC, damp=0.8), dict(), dict(precision=ugmg.MIXED)])
-def test_calls_that_do_not_wait(kw):
+def test_calls_that_do_not_wait(kw, monkeypatch):
     """Alternating levels and columns, more of them than graphs are kept for,
     solves and new parameters in between, with nothing waiting for the GPU:
     no graph goes while it runs."""
+    monkeypatch.setenv("UGMG_FUSE_ROWS", "0")     # the lower levels' cycles are replayed too
     P = problems.q1(2, 3, 4, problems.KAPPA_JUMP, seed=2)
     calls = [(4, 1), (4, 3), (4, 1), (4, 3), (4, 0), (4, 1), (3, 2), (4, 3), (3, 2), (3, 1), (4, 1), (3, 1), (2, 3),
              (2, 2), (2, 1), (2, 3), (2, 2), (2, 1), (4, 2), (3, 3), (4, 2), (3, 3), (4, 1), (4, 0)]

@@ -1143,6 +1143,32 @@ double iteration_bytes(const ugmg_ctx *ctx, int l, int cycles) {
   return by + d.A.bytes(8) + (double)d.n * d.nb * (4.0 + 4.0 + 16.0 + 16.0 + 4.0) + d.n;
 }
 
+// An FP64 cycle on a level in list order works on the caller's vectors; up to
+// this many values the copies to own_c and own_b and back that a replay takes
+// pay.  From 256^2 on the device takes longer than the host.
+constexpr size_t kOwnCycleValues = 65536;
+// the highest level that a cycle does not launch operation by operation
+int launched_above(const ugmg_ctx *ctx) {
+  const int ft = ctx->fuse_top[ctx->p.precision == UGMG_MIXED ? 1 : 0];
+  return ctx->p.gamma == 1 ? std::max(ctx->bl, ft) : ctx->bl;
+}
+// Does a cycle's replay pay?  hipGraphLaunch costs the host about as much as
+// three launches, so not below about 7 on the levels above the base level and
+// those in k_coarse_down and k_coarse_up.  2D cycles of several contexts at
+// once, launched / replayed: none such (33^2) Jacobi 25 / 50 us, GS 33 / 54;
+// 5 (65^2, V(1,1) Jacobi) 47 / 52, mixed 45 / 59, 7 (V(2,2)) 55 / 53, 9
+// (V(3,3)) 63 / 54, 10 (97^2, V(1,1)) 65 / 56.
+bool replay_pays(const ugmg_ctx *ctx, int level) {
+  int n = 0;
+  for (int l = launched_above(ctx) + 1; l <= level; ++l) {
+    auto steps = [&](int nu, bool post) {
+      return sm_kind(ctx, post) == UGMG_SMOOTH_GS ? nu * std::max(ctx->dev[l].ncolors, 1) : nu;
+    };
+    n += steps(ctx->p.nu1, false) + steps(ctx->p.nu2, true) + 3;
+  }
+  return n >= 7;
+}
+
 // The graph that this call's cycle is to be replayed from, or null.  It is
 // recorded by the second call with the same level, columns and c
 // (own_cycle's): a launch per operation takes the host 2.3 to 3 us, as long
@@ -1152,7 +1178,7 @@ double iteration_bytes(const ugmg_ctx *ctx, int l, int cycles) {
 // launches.
 int iter_graph(ugmg_ctx *ctx, int level, const double *c, ugmg_ctx::IterGraph *&out) {
   out = nullptr;
-  if (!can_capture(ctx)) return 0;
+  if (!can_capture(ctx) || !replay_pays(ctx, level)) return 0;
   hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
   HIPCHK(hipStreamIsCapturing(ctx->stream, &cs));
   if (cs != hipStreamCaptureStatusNone) return 0;
@@ -1202,23 +1228,6 @@ int own_cycle(ugmg_ctx *ctx, int level, double *c, double *b, ugmg_ctx::IterGrap
   }
   HIPCHK(hipGraphLaunch(ig->g, ctx->stream));
   return 0;
-}
-
-// Is an FP64 cycle on a level in list order, which works on the caller's
-// vectors, worth the copies to own_c and own_b and back that a replay takes?
-// Jacobi cycles of 2D grids, several contexts at once, launched / replayed:
-// levels in k_coarse_down and k_coarse_up up to the top (33^2) 25 / 50 us; one
-// level above them (65^2) V(1,1) 47 / 52 us, V(2,2) 55 / 53, V(3,3) 63 / 54;
-// two (97^2) V(1,1) 65 / 56.  From 256^2 on the device takes longer than the
-// host.
-constexpr size_t kOwnCycleValues = 65536;
-int launched_above(const ugmg_ctx *ctx) {
-  return ctx->p.gamma == 1 ? std::max(ctx->bl, ctx->fuse_top[0]) : ctx->bl;
-}
-bool replay_pays(const ugmg_ctx *ctx, int level) {
-  const DevLevel &d = ctx->dev[level];
-  return (size_t)d.n * d.nb <= ctx->own_n &&
-         (level - launched_above(ctx)) * (ctx->p.nu1 + ctx->p.nu2 + 3) >= 7;
 }
 
 // ------------------------------------------------------------ BCGSSolver
@@ -1964,7 +1973,7 @@ int prep_device(ugmg_ctx *ctx, PrepState &ps) {
       fill(c32[l], float());
     }
     size_t own = 0;
-    for (int l = launched_above(ctx) + 1; l <= level; ++l) {
+    for (int l = std::max(bl, ctx->p.gamma == 1 ? ctx->fuse_top[0] : bl) + 1; l <= level; ++l) {
       const size_t nv = (size_t)ctx->dev[l].n * ctx->dev[l].nb;
       if (!ctx->dev[l].perm && !ctx->grouped && nv <= kOwnCycleValues) own = std::max(own, nv);
     }
@@ -2698,7 +2707,8 @@ int ugmg_iter(ugmg_ctx *ctx, int level, double *c, double *b) {
   const bool mixed = ctx->p.precision == UGMG_MIXED, list = !d.perm && !mixed;
   double *oc = mixed ? nullptr : list ? ctx->own_c : d.c, *ob = mixed ? nullptr : list ? ctx->own_b : d.b;
   ugmg_ctx::IterGraph *ig = nullptr;
-  if ((!list || replay_pays(ctx, level)) && (rc = iter_graph(ctx, level, oc, ig))) return rc;
+  const bool fits = !list || (size_t)d.n * d.nb <= ctx->own_n;
+  if (fits && (rc = iter_graph(ctx, level, oc, ig))) return rc;
   if (mixed) {
     to_dev<float, double>(ctx, level, b, d.vs, d.b32);
     if ((rc = own_cycle(ctx, level, oc, ob, ig))) return rc;
