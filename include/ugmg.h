@@ -263,7 +263,13 @@ int ugmg_interpolate(ugmg_ctx *ctx, int level, double *to_fine,
 /* ---- base solver: ls($m,$red,$abslimit) over ex, on the base level ----- */
 int ugmg_base_solve(ugmg_ctx *ctx, double *c, double *b);
 
-/* ---- NP_ITER: one lmgc cycle on `level`: c := correction, b -= A c ----- */
+/* ---- NP_ITER: one lmgc cycle on `level`: c := correction, b -= A c -----
+ * Asynchronous on the context's stream.  With a GS smoother or MIXED, and for
+ * batches, the level's own b is overwritten: on a locally refined hierarchy
+ * the next cycle on level + 1 adds to it where VNCLASS < 2 (FP64 Jacobi
+ * cycles leave it alone).  With use_graph, cycles of enough launches are
+ * replayed from the second call with a level and column count on; the first
+ * call with another one or after ugmg_set_params is launched.              */
 int ugmg_iter(ugmg_ctx *ctx, int level, double *c, double *b);
 int ugmg_iter_host(ugmg_ctx *ctx, int level, double *c, double *b);
 

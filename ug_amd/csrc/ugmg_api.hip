@@ -1356,11 +1356,17 @@ int launch_bcgs_iteration(ugmg_ctx *ctx, int level, bool use_iter, int restart, 
 // 9^3 (187e6) 12.3 / 5.6, 11^3 59 / 13
 constexpr double kBaseDeviceWork = 5.0e7;
 
-// the largest level that k_coarse_down and k_coarse_up take.  A pass over a
-// level's slabs through one CU overtakes the launches it saves at a few
-// thousand rows: 2D Poisson solve 1756 us with none, 1407 us up to 17^2, 1342
-// us up to 33^2, 1633 us up to 65^2; serving 32.0 ms with none, 29.9 ms up to
-// 9^3, 29.7 ms up to 17^3
+// The largest level that k_coarse_down and k_coarse_up take.  A pass over a
+// level's slabs through one CU overtakes the launches that it saves; where,
+// depends on the launches (GS has one a colour, Jacobi one a step), on the
+// entries and on the columns, which have a CU each.  One V(2,2) level above
+// the base level, launches / one workgroup, us: GS 33^2 (1089 rows) 71 / 52,
+// 41^2 73 / 59, 49^2 (2401) 73 / 67, 57^2 (3249) 76 / 77, with 8 columns 108 /
+// 89, 65^2 115 / 106; 9^3 139 / 86, 11^3 (1331) 138 / 99, 15^3 (3375) 144 /
+// 141, 17^3 144 / 171, with 8 columns 171 / 178.  Jacobi 33^2 41 / 44, 41^2
+// 42 / 50, 65^2 43 / 86; 9^3 48 / 46, 11^3 49 / 59.  So the line is where
+// Jacobi breaks even; several levels down to a small base level (33^2 to
+// 3^2: 97 / 73) and contexts that share the host gain more.
 constexpr int kCoarseRows = 1200;
 
 // FULLREFINELEVEL of the levels set up to `level` (SetSurfaceClasses,

@@ -332,14 +332,17 @@ __global__ __launch_bounds__(64) void k_band_inverse(const double *__restrict__ 
 // Backward the order of the terms (ascending from the row's own successor)
 // makes each column one chain: one wave walks it, 16 terms a time with the
 // operands of the next 16 on their way from LDS and the next row of U on its
-// way from memory.  That chain bounds the kernel (29 cycles a term).
+// way from memory.  That wave bounds the kernel: 29 cycles a term, of which
+// the dependent subtraction takes 8; the reads and products that it issues
+// besides take the rest, while the other three waves are done.
 // Terms a chunk covers beyond the row's range are discarded by a select.
 //
 // Elimination fills a row only from its first to its last column of the
 // matrix' own envelope: lfirst[q] is the first column of rows 16 q .. 16 q +
 // 15 of L, ulast[i] the last of row i of U (about half of bw on the average
 // in BFS order, whose level sets grow and shrink); the terms outside are
-// zeros.
+// zeros.  (Zero times a solution entry: where one overflowed, the host's
+// substitutions give NaN in more places than these.)
 // 17^3 base level (n 4913, bw 907), 246 workgroups of 20 columns: 175 -> 43 ms
 // (forward 7, backward 36).
 constexpr int kCh = 16;

@@ -1540,9 +1540,12 @@ void launch_galerkin(hipStream_t st, int nc, int bb, const int *ptp, const int *
 // and the rest the chain kernel arguments -> slice header -> entries ->
 // gather; here an operation ends in a workgroup barrier, the vectors are in
 // LDS, and headers stay in the scalar cache.  The workgroup reads the slabs
-// through one CU (about 64 bytes a cycle), which bounds the larger levels.
-// Every row is formed as in the separate kernels, in the same order: the
-// same bits.  V(1,1) Jacobi cycle on 65^2, levels up to 33^2 here: 101 -> 51 us.
+// through one CU (about 64 bytes a cycle), which bounds the larger levels;
+// on the smaller ones each pass waits for its entries from memory (about 1.7
+// us a pass: 20 passes of a V(1,1) Jacobi cycle on 33^2 take 35 us).  Every
+// row is formed as in the separate kernels, in the same order: the same bits.
+// V(2,2) GS cycle on 33^2, base level 5^2: 169 -> 93 us; on 65^2, levels up to
+// 33^2 here: 221 -> 148 us.
 //
 // The kernels store between their passes, so what they read through level
 // and slab pointers would be loaded per lane; it does not change while they
